@@ -219,6 +219,116 @@ struct Layout {
   int64_t max_pages, page_log2, num_pages;
 };
 
+// ---- work-balanced paged calls (decode_balanced_kernel) ----
+//
+// A span shorter than MIN_SPAN tiles per wave only adds pieces to merge.
+// Starting a row costs a wave about as much as streaming ROW_COST tiles (its
+// query and page ids fetched, the row before it totalled): with 0 / 2 / 4 / 8,
+// batch 60 of 100-6000 tokens, int4 D 128: 39.2 / 36.3 / 34.8 / 34.4 us, fp16
+// batch 32 of 120-7700: 52.5 / 51.2 / 51.0 / 51.4 us. With few rows per wave
+// it would only upset an even cut, so it is then 0.
+constexpr int MIN_SPAN = 2;
+constexpr int ROW_COST = 4;
+
+int balanced_wg(int fmt, int64_t D, int hg, int64_t W) {
+  const int most = balanced_nw(fmt, (int)D, hg);
+  return W < most ? (int)W : most;
+}
+// Workgroups of a call: as many as are resident (more only queue behind them:
+// twice as many measured 8-10 us slower at every size), a multiple of 8.
+int64_t balanced_spans(int fmt, int hg, int64_t rows, int64_t N, int64_t D, int64_t W, int cus) {
+  const int64_t nw = balanced_wg(fmt, D, hg, W);
+  const int64_t resident = (int64_t)cus * (balanced_waves(fmt, (int)D, hg) * 4 / nw);
+  const int64_t units = rows * ((N + 15) / 16 + ROW_COST);
+  int64_t n = (units + MIN_SPAN * nw - 1) / (MIN_SPAN * nw);
+  if (n > resident) n = resident;
+  if (n > BALANCED_MAX_SPANS) n = BALANCED_MAX_SPANS;
+  return (n + 7) & ~(int64_t)7;
+}
+size_t balanced_bytes(int64_t spans, int hg, int64_t D) {
+  return 2 * (size_t)spans * (size_t)entry_floats((int)D, hg) * sizeof(float) + 128;  // 128: to a cache line
+}
+
+// Waves per workgroup of a single-block call (W is a maximum). Workgroups of 4
+// waves with four times as many work items as CUs, and
+// with more unsplit work items than CUs for rows under 256 bytes (128-byte
+// rows from one per CU on): several share a CU and hide each other's
+// memory latency, where 8-wave ones fit one per CU at these kernels'
+// register counts and leave a partial round (same-box A/B on MI355X at
+// N 4096, 384 / 512 / 768 KV rows: int8 at D 128 -9 / -8 / -6 %, int4
+// -11 / -9 / -9 %, fp8 and int8 at D 64 -8 to -13 %, fp16 at D 64 -13 /
+// -3 / -6 %, int4 at D 64 within 3 %; at 256 rows int8 / fp8 at D 128 and
+// fp16 at D 64 -6 to -8 %, while 64-byte rows are faster with 8 waves;
+// fp16 / bf16 rows of 256 bytes run 1-2 % slower with 4 waves and keep 8
+// below 4 x CUs).
+int64_t waves_for(int fmt, int64_t D, int64_t nblocks, int64_t S, int64_t W, int cus) {
+  const int64_t rowb = row_bytes_of(fmt, D);
+  const bool many = nblocks >= 4LL * cus ||
+                    (S == 1 && rowb < 256 && (nblocks > cus || (rowb == 128 && nblocks == cus)));
+  return many && W > 4 ? 4 : W;
+}
+
+// Whether a paged call takes the work-balanced kernel. The lengths are on the
+// device, so the rule weighs what the call can hold at most: tiles per wave of
+// the resident grid. Few tiles leave the fixed costs (finding the wave's place,
+// a device-scope merge: ~4 us) uncovered; and where one workgroup per (row,
+// split) loads the GPU evenly, sequences of one length need no balancing, so
+// there the line is higher. Measured against that path (fp16 D 128, 8 KV
+// heads, equal lengths / lengths spread 1:20; tiles per wave): batch 16 of
+// 3000 tokens (11.8) 36.0 -> 39.6 / 27.0 -> 22.7 us, 64 of 1500 (23.5) 66.2 ->
+// 68.5 / 37.5 -> 32.3 us, 120 of 3000 (88) 239 -> 229 us; with a last round
+// mostly empty, batch 40 of 1500 (14.7): 55.7 -> 49.5 / 28.2 -> 23.7 us. int4
+// at D 128 crosses later (32 of 8000, 41.7: 67.7 -> 66.3 us), and wide head
+// groups have more to merge.
+bool balanced_pays(int fmt, int hg, int64_t B, int64_t rows, int64_t N, int64_t D, int64_t S, int64_t W,
+                   size_t ws_bytes, int cus) {
+  // 32-bit positions on the line, one arrival counter per row
+  if (B > BALANCED_MAX_SEQS || rows > MAX_SPLIT_GROUPS || rows * ((N + 15) / 16 + 16) >= (int64_t(1) << 30))
+    return false;
+  if (ws_bytes < balanced_bytes(balanced_spans(fmt, hg, rows, N, D, W, cus), hg, D)) return false;
+  const int waves = balanced_waves(fmt, (int)D, hg) * 4;  // per CU
+  const int64_t wgs = rows * S;
+  const int64_t nw = waves_for(fmt, D, wgs, S, W, cus);
+  const int64_t round = (int64_t)cus * (waves > nw ? waves / nw : 1);  // workgroups side by side
+  // evenly: one round that keeps 6 waves on every CU, or rounds 0.9 full
+  const bool even = wgs <= round ? wgs * nw >= 6LL * cus : wgs * 10 >= (wgs + round - 1) / round * round * 9;
+  const int least = even ? (fmt == KV_I4 && D == 128 ? 36 : 28) : (hg >= 8 ? 16 : 10);
+  return rows * ((N + 15) / 16) >= least * (int64_t)cus * waves;
+}
+
+int run_balanced(const PartialParams& base, int fmt, int hg, int64_t B, int64_t N, int64_t D, int64_t W, void* ws,
+                 hipStream_t st, int cus) {
+  if (!aligned(ws, 16)) return fail(FQKV_ERR_ARG, "workspace must be 16-byte aligned");
+  BalancedParams p{};
+  static_cast<PartialParams&>(p) = base;
+  const int64_t rows = B * p.hkv * p.ngroups;
+  const int nw = balanced_wg(fmt, D, hg, W);
+  // heads sharing a 128-byte line of a token: rows under 128 bytes, token-major
+  const int64_t rowb = row_bytes_of(fmt, D);
+  int k = 0;
+  while ((2 << k) * rowb <= 128 && p.hkv % (2 << k) == 0 && p.kv_ts >= (2 << k) * rowb) ++k;
+  if (p.kv_hs != rowb) k = 0;
+  int64_t spans = (balanced_spans(fmt, hg, rows, N, D, W, cus) >> k) & ~(int64_t)7;
+  if (spans == 0) {
+    k = 0;
+    spans = balanced_spans(fmt, hg, rows, N, D, W, cus);
+  }
+  p.nb = (int)B;
+  p.nspan = (int)spans;
+  p.hk = k;
+  p.rg = (p.hkv >> k) * p.ngroups;
+  p.row_cost = rows * 16 > (spans * nw << k) ? ROW_COST : 0;
+  p.min_span = MIN_SPAN * nw;
+  p.direct = 0;
+  p.m_part = (float*)(((uintptr_t)ws + 127) & ~(uintptr_t)127);
+  p.slot = merge_slot(st, rows, &p.xcd_ok);
+  int xcd_local = 0;
+  const hipError_t e = launch_balanced(fmt, (int)D, hg, p, nw, st, &xcd_local);
+  if (e != hipSuccess) return hip_fail(e, "launch: balanced kernel");
+  record_protocol(2, p.slot, xcd_local);
+  return FQKV_OK;
+}
+
 int run_decode(int fmt, const void* q, const void* K, const void* V, const void* Ks,
                const void* Vs, void* o, int64_t rows, int64_t G, int64_t N, int64_t D, int64_t W,
                void* ws, size_t ws_bytes, hipStream_t st, const Layout* L = nullptr) {
@@ -229,6 +339,9 @@ int run_decode(int fmt, const void* q, const void* K, const void* V, const void*
   const int64_t ngroups = (G + hg - 1) / hg;
   const int64_t heads = rows * G;
   int64_t S = splits_for(rows, G, N, fmt, W, cus);
+  const bool balance = L && L->page_table &&
+                       balanced_pays(fmt, hg, rows / L->hkv, rows * ngroups, N, D, S, W, ws ? ws_bytes : 0, cus);
+  if (balance) S = 1;
   if (S > 1 && (ws == nullptr || scratch_bytes(heads, S, D) > ws_bytes)) {
     int64_t fit = ws ? (int64_t)(ws_bytes / scratch_bytes(heads, 1, D)) : 0;
     while (fit >= 2 && scratch_bytes(heads, fit, D) > ws_bytes) --fit;
@@ -249,7 +362,14 @@ int run_decode(int fmt, const void* q, const void* K, const void* V, const void*
   p.N = (int)N;
   p.S = (int)S;
   p.chunk = (int)((N + S - 1) / S);
-  if (L && L->page_table) p.chunk = (p.chunk + 15) & ~15;  // a paged tile must not cross a page
+  if (L && L->page_table) {
+    p.chunk = (p.chunk + 15) & ~15;  // a paged tile must not cross a page
+    // In one round of workgroups a sequence shorter than the call allows is
+    // better cut into S parts of its own (a static cache of 2048, 1100 filled,
+    // batch 16, int4 D 64: 14.2 -> 12.8 us with its append); with more
+    // workgroups than CUs the parts it would leave empty spare a second round.
+    p.own_chunk = nblocks <= cus;
+  }
   p.ngroups = (int)ngroups;
   p.scale = 1.0f / sqrtf((float)D);
   p.c = p.scale * 1.4426950408889634f;
@@ -270,6 +390,7 @@ int run_decode(int fmt, const void* q, const void* K, const void* V, const void*
     p.page_log2 = (int)L->page_log2;
     p.num_pages = (int)L->num_pages;
   }
+  if (balance) return run_balanced(p, fmt, hg, rows / L->hkv, N, D, W, ws, st, cus);
   if (!p.direct) {
     float* f = (float*)ws;
     p.m_part = f;
@@ -277,21 +398,7 @@ int run_decode(int fmt, const void* q, const void* K, const void* V, const void*
     p.o_part = f + acc_offset_floats(heads, S);
     p.slot = merge_slot(st, rows * ngroups, &p.xcd_ok);
   }
-  // Workgroups of 4 waves with four times as many work items as CUs, and
-  // with more unsplit work items than CUs for rows under 256 bytes (128-byte
-  // rows from one per CU on): several share a CU and hide each other's
-  // memory latency, where 8-wave ones fit one per CU at these kernels'
-  // register counts and leave a partial round (same-box A/B on MI355X at
-  // N 4096, 384 / 512 / 768 KV rows: int8 at D 128 -9 / -8 / -6 %, int4
-  // -11 / -9 / -9 %, fp8 and int8 at D 64 -8 to -13 %, fp16 at D 64 -13 /
-  // -3 / -6 %, int4 at D 64 within 3 %; at 256 rows int8 / fp8 at D 128 and
-  // fp16 at D 64 -6 to -8 %, while 64-byte rows are faster with 8 waves;
-  // fp16 / bf16 rows of 256 bytes run 1-2 % slower with 4 waves and keep 8
-  // below 4 x CUs). W is a maximum.
-  const int64_t rowb = row_bytes_of(fmt, D);
-  const bool many = nblocks >= 4LL * cus ||
-                    (S == 1 && rowb < 256 && (nblocks > cus || (rowb == 128 && nblocks == cus)));
-  const int64_t nw = (many && W > 4) ? 4 : W;
+  const int64_t nw = waves_for(fmt, D, nblocks, S, W, cus);
   int xcd_local = 0;
   hipError_t e = launch_partial(fmt, (int)D, hg, p, (int)nblocks, (int)nw, st, &xcd_local);
   if (e != hipSuccess) return hip_fail(e, "launch: partial kernel");
@@ -491,8 +598,17 @@ int64_t fqkv_choose_splits(int64_t rows, int64_t G, int64_t N, int64_t D, int kv
 }
 
 size_t fqkv_workspace_bytes(int64_t rows, int64_t G, int64_t N, int64_t D, int kv_format, int64_t W) {
-  const int64_t S = fqkv_choose_splits(rows, G, N, D, kv_format, W);
-  return S > 1 ? scratch_bytes(rows * G, S, D) : 0;
+  int cus = 256;
+  if (device_cus(&cus) != FQKV_OK) cus = 256;
+  if (rows < 1 || G < 1 || N < 1) return 0;
+  const int64_t S = splits_for(rows, G, N, kv_format, W, cus);
+  const size_t split = S > 1 ? scratch_bytes(rows * G, S, D) : 0;
+  const int hg = choose_hg(G, kv_format);
+  const int64_t work_rows = rows * ((G + hg - 1) / hg);
+  // (a paged call of these sizes may take the work-balanced kernel)
+  const size_t spans = balanced_bytes(balanced_spans(kv_format, hg, work_rows, N, D, W, cus), hg, D);
+  if (!balanced_pays(kv_format, hg, 1, work_rows, N, D, S, W, spans, cus)) return split;
+  return split > spans ? split : spans;
 }
 
 int fqkv_decode_attn_fp16_mw(const void* q, const void* K, const void* V, void* o, int64_t B,

@@ -76,7 +76,8 @@ constexpr float LOG2E = 1.4426950408889634f;
 // host (or, with bytes = SIZE_MAX, clears).
 #ifdef FQKV_TIMELINE
 constexpr int TIMELINE_BLOCKS = 4096;
-__device__ unsigned long long g_timeline[TIMELINE_BLOCKS][NW_MAX][16];
+constexpr int TIMELINE_WAVES = NW_MAX;  // waves past it leave no stamps
+__device__ unsigned long long g_timeline[TIMELINE_BLOCKS][TIMELINE_WAVES][16];
 // The stamp takes its own copy of the workgroup id (an asm move the compiler
 // cannot merge with the kernel's uses): indexing g_timeline with blockIdx.x
 // itself under the lane-0 branch made the compiler carry the id in a vector
@@ -88,11 +89,12 @@ __device__ unsigned long long g_timeline[TIMELINE_BLOCKS][NW_MAX][16];
     uint32_t blk_;                                                                                 \
     asm volatile("s_mov_b32 %0, %1" : "=s"(blk_) : "s"(blockIdx.x));                              \
     const unsigned long long t_ = __builtin_amdgcn_s_memrealtime();                                \
-    if ((threadIdx.x & 63) == 0 && blk_ < TIMELINE_BLOCKS) g_timeline[blk_][threadIdx.x >> 6][stage] = t_; \
+    if ((threadIdx.x & 63) == 0 && blk_ < TIMELINE_BLOCKS && (threadIdx.x >> 6) < TIMELINE_WAVES)                 \
+      g_timeline[blk_][threadIdx.x >> 6][stage] = t_; \
   } while (0)
 extern "C" int fqkv_timeline_read(void* host, size_t bytes) {
   if (bytes == (size_t)-1) {
-    static unsigned long long z[TIMELINE_BLOCKS][NW_MAX][16];
+    static unsigned long long z[TIMELINE_BLOCKS][TIMELINE_WAVES][16];
     return (int)hipMemcpyToSymbol(HIP_SYMBOL(g_timeline), z, sizeof(z));
   }
   return (int)hipMemcpyFromSymbol(host, HIP_SYMBOL(g_timeline), bytes);
@@ -342,11 +344,44 @@ __device__ __forceinline__ auto pick(const uint32_t (&m)[4], Fn f) {
 // bookkeeping.
 // CPOL: cache policy of the partial loads (CPOL_SC1 for partials that other
 // workgroups of the same launch stored at device scope).
+// A: where the partials of split s lie. SplitAddr is the reference's scratch
+// layout; PieceAddr is the work-balanced kernel's (below).
 // s_w: 64 floats per wave (16-byte aligned rows); s_red: 65 floats per wave.
-template <int D, int CPOL>
-__device__ __forceinline__ void merge_splits(const float* __restrict__ m_part, const float* __restrict__ l_part,
-                                             const float* __restrict__ o_part, _Float16* __restrict__ o,
-                                             size_t h0, int nh, int S, float (*s_w)[64], float (*s_red)[65]) {
+struct SplitAddr {
+  const float *m, *l, *o;  // m[h S + s], l likewise, o[(h S + s) D + d]
+  size_t h0;
+  int S;
+  __device__ __forceinline__ const float* mrow(int h) const { return m + (h0 + h) * S; }
+  __device__ __forceinline__ const float* lrow(int h) const { return l + (h0 + h) * S; }
+  template <int D>
+  __device__ __forceinline__ const float* orow(int h) const { return o + (h0 + h) * S * D; }
+  // floats from one entry to the next, of m and l and of o
+  __device__ __forceinline__ uint32_t mstep() const { return 1; }
+  template <int D>
+  __device__ __forceinline__ uint32_t ostep() const { return D; }
+  __device__ __forceinline__ uint32_t at(uint32_t s) const { return s; }
+};
+// Pieces of a row as the work-balanced kernel stores them, entry by entry
+// (entry_floats: m of up to 16 heads, l of up to 16, then HG rows of D; a
+// multiple of 128 bytes, so no two entries share a cache line and each line is
+// written and read by one protocol). Workgroup i owns entries 2i (a piece that
+// starts inside its row) and 2i + 1 (one that starts it); a row's pieces are
+// entry 2a + 1, then 2 (a + s). base: entry 2a + 1.
+template <int D, int HG>
+struct PieceAddr {
+  const float* base;
+  __device__ __forceinline__ const float* mrow(int h) const { return base + h; }
+  __device__ __forceinline__ const float* lrow(int h) const { return base + 16 + h; }
+  template <int>
+  __device__ __forceinline__ const float* orow(int h) const { return base + 32 + h * D; }
+  __device__ __forceinline__ uint32_t mstep() const { return entry_floats(D, HG); }
+  template <int>
+  __device__ __forceinline__ uint32_t ostep() const { return entry_floats(D, HG); }
+  __device__ __forceinline__ uint32_t at(uint32_t s) const { return s == 0 ? 0u : 2u * s - 1u; }
+};
+template <int D, int CPOL, typename A>
+__device__ __forceinline__ void merge_splits(const A& ad, _Float16* __restrict__ o, size_t h0, int nh, int S,
+                                             float (*s_w)[64], float (*s_red)[65]) {
   constexpr int DB = D / 64;  // units per head
   constexpr int CHK = 32;     // splits per chunk: 8 loads of 4 splits per lane
   constexpr int NJ = CHK / 4;
@@ -387,14 +422,16 @@ __device__ __forceinline__ void merge_splits(const float* __restrict__ m_part, c
     if (wv < units) {
       const int h = wv / DB;
       const size_t hrow = h0 + h;
-      const rsrc_t rM = make_rsrc(m_part + hrow * S, (uint32_t)S * 4u);
-      const rsrc_t rL = make_rsrc(l_part + hrow * S, (uint32_t)S * 4u);
-      const rsrc_t rO = make_rsrc(o_part + hrow * S * D + (wv - h * DB) * 64, (uint32_t)(S - 1) * D * 4u + 256u);
-      const float m0 = ld(rM, 4u * (uint32_t)lane);
-      const float l0 = ld(rL, 4u * (uint32_t)lane);
+      const uint32_t last = ad.at(S - 1);
+      const rsrc_t rM = make_rsrc(ad.mrow(h), last * ad.mstep() * 4u + 4u);
+      const rsrc_t rL = make_rsrc(ad.lrow(h), last * ad.mstep() * 4u + 4u);
+      const rsrc_t rO = make_rsrc(ad.template orow<D>(h) + (wv - h * DB) * 64, last * ad.template ostep<D>() * 4u + 256u);
+      const uint32_t lo4 = ad.at(lane) * ad.mstep() * 4u;
+      const float m0 = ld(rM, lo4);
+      const float l0 = ld(rL, lo4);
       fl4_t ov[NJ];
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) ov[j] = ld4(rO, (uint32_t)((4 * j + kr) * D * 4) + qo);  // zero past split S - 1
+      for (int j = 0; j < NJ; ++j) ov[j] = ld4(rO, ad.at(4 * j + kr) * ad.template ostep<D>() * 4u + qo);  // zero past split S - 1
       float M = wave_max(lane < S ? m0 : -INFINITY);
       FQKV_STAMP(8);  // merge: maximum over the splits known
       if (M == -INFINITY) M = 0.0f;  // every split empty: all weights 0
@@ -411,6 +448,50 @@ __device__ __forceinline__ void merge_splits(const float* __restrict__ m_part, c
         acc4.w = fmaf(wk, ov[j].w, acc4.w);
       }
       emit(acc4, L, o + hrow * D + (wv - h * DB) * 64);
+    }
+    return;
+  }
+  if (S <= CHK) {
+    // More units than waves: a wave's units two at a time, both units' loads
+    // out before either is used (one memory round trip per pair).
+    for (int u0 = wv; u0 < units; u0 += 2 * nw) {
+      const int two = u0 + nw < units ? 2 : 1;
+      fl4_t ov[2][NJ];
+      float m0[2], l0[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int u = u0 + (k < two ? k * nw : 0);
+        const int h = u / DB;
+        const uint32_t last = ad.at(S - 1);
+        const rsrc_t rM = make_rsrc(ad.mrow(h), last * ad.mstep() * 4u + 4u);
+        const rsrc_t rL = make_rsrc(ad.lrow(h), last * ad.mstep() * 4u + 4u);
+        const rsrc_t rO = make_rsrc(ad.template orow<D>(h) + (u - h * DB) * 64, last * ad.template ostep<D>() * 4u + 256u);
+        const uint32_t lo4 = ad.at(lane) * ad.mstep() * 4u;
+        m0[k] = ld(rM, lo4);
+        l0[k] = ld(rL, lo4);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) ov[k][j] = ld4(rO, ad.at(4 * j + kr) * ad.template ostep<D>() * 4u + qo);
+      }
+      auto finish = [&](int u, float mk, float lk, const fl4_t (&v)[NJ]) __attribute__((always_inline)) {
+        const int h = u / DB;
+        float M = wave_max(lane < S ? mk : -INFINITY);
+        if (M == -INFINITY) M = 0.0f;  // every split empty: all weights 0
+        const float wt = lane < S ? fast_exp2((mk - M) * LOG2E) : 0.0f;
+        s_w[wv][lane] = wt;
+        const float L = wave_sum(wt * lk);
+        fl4_t acc4 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const float wk = s_w[wv][4 * j + kr];
+          acc4.x = fmaf(wk, v[j].x, acc4.x);
+          acc4.y = fmaf(wk, v[j].y, acc4.y);
+          acc4.z = fmaf(wk, v[j].z, acc4.z);
+          acc4.w = fmaf(wk, v[j].w, acc4.w);
+        }
+        emit(acc4, L, o + (h0 + h) * D + (u - h * DB) * 64);
+      };
+      finish(u0, m0[0], l0[0], ov[0]);
+      if (two == 2) finish(u0 + nw, m0[1], l0[1], ov[1]);
     }
     return;
   }
@@ -432,21 +513,22 @@ __device__ __forceinline__ void merge_splits(const float* __restrict__ m_part, c
     float L = 0.0f;
     if (live) {
       const size_t hrow = h0 + h;
-      const rsrc_t rM = make_rsrc(m_part + hrow * S, (uint32_t)S * 4u);
-      const rsrc_t rL = make_rsrc(l_part + hrow * S, (uint32_t)S * 4u);
-      // split start + i, dims 4q .. 4q+3 at byte i D 4 + qo; the record ends
-      // with the slice's last split's 64 dims
-      const rsrc_t rO = make_rsrc(o_part + (hrow * S + start) * D + db * 64,
-                                  (uint32_t)(end - start - 1) * D * 4u + 256u);
-      const uint32_t lo4 = (uint32_t)lane * 4u;
-      const float m0 = ld(rM, lo4);
-      const float l0 = ld(rL, lo4);
+      const uint32_t last = ad.at(S - 1);
+      const rsrc_t rM = make_rsrc(ad.mrow(h), last * ad.mstep() * 4u + 4u);
+      const rsrc_t rL = make_rsrc(ad.lrow(h), last * ad.mstep() * 4u + 4u);
+      // split s, dims 4q .. 4q+3 at entry at(s); the record ends with the
+      // slice's last split's 64 dims
+      const rsrc_t rO = make_rsrc(ad.template orow<D>(h) + db * 64, ad.at(end - 1) * ad.template ostep<D>() * 4u + 256u);
+      auto ml = [&](int s0) { return ad.at(s0 + lane) * ad.mstep() * 4u; };
+      auto od = [&](int s0) { return ad.at(s0 + kr) * ad.template ostep<D>() * 4u + qo; };
+      const float m0 = ld(rM, ml(0));
+      const float l0 = ld(rL, ml(0));
       fl4_t ov[NJ];
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) ov[j] = ld4(rO, (uint32_t)((4 * j + kr) * D * 4) + qo);
+      for (int j = 0; j < NJ; ++j) ov[j] = ld4(rO, od(start + 4 * j));
       float M = lane < S ? m0 : -INFINITY;
       for (int s0 = 64; s0 < S; s0 += 64) {
-        const float mm = ld(rM, lo4 + (uint32_t)s0 * 4u);
+        const float mm = ld(rM, ml(s0));
         M = fmaxf(M, s0 + lane < S ? mm : -INFINITY);
       }
       M = wave_max(M);
@@ -456,8 +538,8 @@ __device__ __forceinline__ void merge_splits(const float* __restrict__ m_part, c
         if (c0 == start || (c0 & 63) == 0) {  // weights of splits 64 b .. 64 b + 63 in this slice
           float mm = m0, ll = l0;
           if (b > 0) {
-            mm = ld(rM, lo4 + (uint32_t)b * 256u);
-            ll = ld(rL, lo4 + (uint32_t)b * 256u);
+            mm = ld(rM, ml(64 * b));
+            ll = ld(rL, ml(64 * b));
           }
           const int sk = 64 * b + lane;
           const float w = sk >= start && sk < end ? fast_exp2((mm - M) * LOG2E) : 0.0f;
@@ -478,7 +560,7 @@ __device__ __forceinline__ void merge_splits(const float* __restrict__ m_part, c
         if (c1 < end) {
           fl4_t nv[NJ];
 #pragma unroll
-          for (int j = 0; j < NJ; ++j) nv[j] = ld4(rO, (uint32_t)((c1 - start + 4 * j + kr) * D * 4) + qo);
+          for (int j = 0; j < NJ; ++j) nv[j] = ld4(rO, od(c1 + 4 * j));
           accumulate(ov);
 #pragma unroll
           for (int j = 0; j < NJ; ++j) ov[j] = nv[j];
@@ -560,10 +642,11 @@ __device__ __forceinline__ float tree_sum(const float (&v)[N]) {
   }
 }
 
-template <int D, int HG, int NWC>
-__device__ __forceinline__ void merge_waves_emit(const PartialParams& p, const float (*s_o)[HG][opitch<D>()],
-                                                 const float (*s_m)[NW_MAX], const float (*s_l)[NW_MAX],
-                                                 size_t qrow0, int hcnt, int s) {
+// put(head, element d, M, L, O): the head's maximum (in score units), sum of
+// weights and four accumulators.
+template <int D, int HG, int NWC, typename Put>
+__device__ __forceinline__ void merge_waves(float c, const float (*s_o)[HG][opitch<D>()], const float (*s_m)[NW_MAX],
+                                            const float (*s_l)[NW_MAX], int hcnt, Put put) {
   static_assert(NWC == 2 || NWC == 4 || NWC == 8, "waves per workgroup");
   for (int idx = 4 * (int)threadIdx.x; idx < hcnt * D; idx += 4 * (int)blockDim.x) {
     const int h = idx / D;
@@ -585,7 +668,7 @@ __device__ __forceinline__ void merge_waves_emit(const PartialParams& p, const f
     float wj[NWC], wl[NWC];
 #pragma unroll
     for (int j = 0; j < NWC; ++j) {
-      wj[j] = fast_exp2((mw[j] - Mu) * p.c);
+      wj[j] = fast_exp2((mw[j] - Mu) * c);
       wl[j] = wj[j] * lw[j];
     }
     const float L = tree_sum<NWC>(wl);
@@ -597,18 +680,27 @@ __device__ __forceinline__ void merge_waves_emit(const PartialParams& p, const f
       O.z = fmaf(wj[ww], a[ww].z, O.z);
       O.w = fmaf(wj[ww], a[ww].w, O.w);
     }
+    put(h, d, M, L, O);
+  }
+}
+
+// Normalised fp16 output of four elements (an empty sequence gives zeros).
+__device__ __forceinline__ void put_output(_Float16* dst, float L, fl4_t O) {
+  const float Ox = O.x, Oy = O.y, Oz = O.z, Ow = O.w;
+  dst[0] = L > 0.0f ? (_Float16)(Ox / L) : (_Float16)0.0f;
+  dst[1] = L > 0.0f ? (_Float16)(Oy / L) : (_Float16)0.0f;
+  dst[2] = L > 0.0f ? (_Float16)(Oz / L) : (_Float16)0.0f;
+  dst[3] = L > 0.0f ? (_Float16)(Ow / L) : (_Float16)0.0f;
+}
+
+template <int D, int HG, int NWC>
+__device__ __forceinline__ void merge_waves_emit(const PartialParams& p, const float (*s_o)[HG][opitch<D>()],
+                                                 const float (*s_m)[NW_MAX], const float (*s_l)[NW_MAX],
+                                                 size_t qrow0, int hcnt, int s) {
+  merge_waves<D, HG, NWC>(p.c, s_o, s_m, s_l, hcnt, [&](int h, int d, float M, float L, fl4_t O) {
     const size_t qh = qrow0 + h;
-    // normalised fp16 output (an empty sequence gives zeros)
-    auto put_out = [&]() {
-      _Float16* dst = p.o + qh * D + d;
-      const float Ox = O.x, Oy = O.y, Oz = O.z, Ow = O.w;
-      dst[0] = L > 0.0f ? (_Float16)(Ox / L) : (_Float16)0.0f;
-      dst[1] = L > 0.0f ? (_Float16)(Oy / L) : (_Float16)0.0f;
-      dst[2] = L > 0.0f ? (_Float16)(Oz / L) : (_Float16)0.0f;
-      dst[3] = L > 0.0f ? (_Float16)(Ow / L) : (_Float16)0.0f;
-    };
     if (p.direct) {
-      put_out();
+      put_output(p.o + qh * D + d, L, O);
     } else {
       const size_t b = qh * p.S + s;
       float* orow = p.o_part + b * D + d;
@@ -644,9 +736,9 @@ __device__ __forceinline__ void merge_waves_emit(const PartialParams& p, const f
       }
       // one split: the workgroup holds the whole result, so it writes the
       // output too and no merge follows (one launch per call)
-      if (p.S == 1) put_out();
+      if (p.S == 1) put_output(p.o + qh * D + d, L, O);
     }
-  }
+  });
 }
 
 // Forces the launch constants into scalar registers at this point (an empty
@@ -671,7 +763,7 @@ __device__ __forceinline__ void pin_sgprs(const PartialParams& p) {
   }
   if constexpr (PAGED) {
     pin_s(p.kv_bs); pin_s(p.page_table); pin_s(p.seq_lens); pin_s(p.max_pages); pin_s(p.page_log2);
-    pin_s(p.num_pages);
+    pin_s(p.num_pages); pin_s(p.own_chunk); pin_s(p.S); pin_s(p.div_S.magic); pin_s(p.div_S.shift);
     if constexpr (QUANT) pin_s(p.sc_bs);
   }
 }
@@ -704,15 +796,39 @@ constexpr int tiles_per_pass() {
   return SHORT ? 2 : ((FMT == KV_I4 && D == 64 && HG == 1 && !PAGED && !PVV) ? 8 : 4);
 }
 
+// A wave's K staging bytes, and where wave w's lie.
+template <typename F>
+constexpr int kstage_bytes() {
+  if constexpr (F::STAGE_K)
+    return F::KSTAGE;
+  else
+    return 0;
+}
+template <typename F>
+__device__ __forceinline__ uint8_t* kstage_of(uint8_t* s, int w) {
+  if constexpr (F::STAGE_K)
+    return s + w * F::KSTAGE;
+  else
+    return nullptr;
+}
+
 // KEEPV: int4 rows token-major without pages (heads sharing cache lines, the
 // launcher's head grouping on), whose V loads go without the non-temporal hint.
 // LAZY (int8 / int4 / fp8 / bf16, each wave one four-tile pass): the query's
 // derived operands are formed, and a pass's scales unpacked, only once the
 // pass's K and V loads are all out (see qprep and the scale loads below);
 // with several passes per wave the registers this keeps live cost occupancy.
-template <int FMT, int D, int HG, bool PAGED, bool PVV = false, bool KEEPV = false, bool SHORT = false,
-          bool LAZY = false>
-__global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialParams p) {
+//
+// stream_rows: one wave's part of a work item. Of tokens lo .. hi - 1 of KV
+// row (b, h) it streams the 16-token tiles tw, tw + tn, ... for query heads
+// qrow0 .. qrow0 + hcnt - 1, and leaves its (m, l, acc) in LDS: m and l of
+// head hh at m_dst / l_dst[hh ml], acc rows of opitch<D>() floats at o_dst.
+// kstage: the wave's F::KSTAGE bytes for fp16 K rows; s_pw: PVV, the wave's
+// weights ([tile][token][head] fp32).
+template <int FMT, int D, int HG, bool PAGED, bool PVV, bool KEEPV, bool SHORT, bool LAZY, bool AHEAD = false>
+__device__ __forceinline__ void stream_rows(const PartialParams& p, int lane, int tw, int tn, int b, int h,
+                                            size_t qrow0, int hcnt, int lo, int hi, float* o_dst, float* m_dst,
+                                            float* l_dst, int ml, uint8_t* kstage, float* s_pw) {
   using F = Fmt<FMT, D>;
   static_assert(!PVV || (FMT == KV_F16 && !PAGED), "P.V on the vector ALUs: fp16, contiguous rows");
   using VG = VGeom<F::ROWB, D>;
@@ -721,52 +837,7 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
   constexpr int U = tiles_per_pass<FMT, D, HG, PAGED, PVV, SHORT>();
   constexpr int VE = VG::VE;   // PV steps per tile
   constexpr int VD = VG::VD;   // dwords per V chunk
-  __shared__ __attribute__((aligned(16))) float s_o[NW_MAX][HG][opitch<D>()];
-  __shared__ __attribute__((aligned(16))) float s_m[HG][NW_MAX];
-  __shared__ __attribute__((aligned(16))) float s_l[HG][NW_MAX];
-  __shared__ __attribute__((aligned(16))) float s_mw[NW_MAX][64];  // in-kernel split merge
-  __shared__ float s_mr[NW_MAX][65];
-  __shared__ int s_last;
-  extern __shared__ __attribute__((aligned(16))) uint8_t s_kstage[];  // fp16 K staging, F::KSTAGE bytes per wave
-
-  FQKV_STAMP(0);  // start
-  const int lane = threadIdx.x & 63;
-  // wave index as a scalar, so tile loops branch per wave, not per lane
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int nw = blockDim.x >> 6;
-  // blockIdx.x = s * nwsg + wsg or wsg * S + s (wsg = r * ngroups + hg),
-  // decomposed with multiply-shift divisions
-  // Every launch constant in one scalar-load round trip: read here, in the
-  // entry block, so the loads leave together (lazily placed, they took four
-  // dependent round trips before the first KV load, and one more before the
-  // epilogue).
-  pin_sgprs<F::QUANT, PAGED>(p);
-  const uint32_t bq = fast_div(blockIdx.x, p.div_blk);
-  const uint32_t br = blockIdx.x - bq * (uint32_t)p.blk_d;
-  uint32_t wsg = p.split_major ? br : bq;
-  const int s = (int)(p.split_major ? bq : br);
-  {
-    // in a block of 2^(hg_k + hg_d) groups, group e 2^hg_d + c becomes row c 2^hg_k + e:
-    // head e of head set c, the set's heads 2^hg_d groups apart (the identity
-    // when hg_k = hg_d = 0; no branch, so the prologue stays one block)
-    const uint32_t k = (uint32_t)p.hg_k, d = (uint32_t)p.hg_d;
-    const uint32_t low = wsg & ((1u << (k + d)) - 1u);
-    wsg = (wsg - low) | ((low & ((1u << d) - 1u)) << k) | (low >> d);
-  }
-  const uint32_t rr = fast_div(wsg, p.div_groups);
-  const int hg = (int)(wsg - rr * (uint32_t)p.ngroups);
-  const int r = (int)rr;
-  // KV row r = (sequence b, KV head h); its tokens sit kv_ts bytes apart
-  const int b = (int)fast_div((uint32_t)r, p.div_hkv);
-  const int h = r - b * p.hkv;
   const uint32_t ts = (uint32_t)p.kv_ts;
-  int nr = p.N;  // tokens of this row
-  if constexpr (PAGED) nr = min(min(p.seq_lens[b], p.N), p.max_pages << p.page_log2);
-  const int lo = s * p.chunk;
-  const int hi = min(lo + p.chunk, nr);
-  const int hbase = hg * HG;
-  const int hcnt = min(HG, p.G - hbase);
-  const size_t qrow0 = (size_t)r * p.G + hbase;
   // base of the row's token 0 (paged: of the row's head within a page)
   const uint8_t* Kr = p.K + (PAGED ? 0 : (size_t)b * p.kv_bs) + (size_t)h * p.kv_hs;
   const uint8_t* Vr = p.V + (PAGED ? 0 : (size_t)b * p.kv_bs) + (size_t)h * p.kv_hs;
@@ -809,7 +880,8 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
   bf8_t qhi[F::BF16 ? F::NKI : 1], qlo[F::BF16 ? F::NKI : 1];
   float qbias = 0.0f;
   constexpr bool QPREP = F::BF16 || F::BIASED;
-  bool qready = !LAZY;
+  constexpr bool LAZYQ = LAZY || (PAGED && AHEAD && F::BIASED);
+  bool qready = !LAZYQ;
   auto qprep = [&]() {
     if constexpr (F::BF16) {
 #pragma unroll
@@ -830,7 +902,7 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
       qbias = F::BIAS * rows4_sum(qs);
     }
   };
-  if constexpr (QPREP && !LAZY) qprep();
+  if constexpr (QPREP && !LAZYQ) qprep();
 
   float m_run = -INFINITY, l_run = 0.0f;  // of column n, over the tokens this lane scored
   float w_run = 0.0f;  // int8 / int4: sum of the lane's PV weights, in acc's units
@@ -844,9 +916,6 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
   for (int h = 0; h < (PVV ? HG : 1); ++h)
 #pragma unroll
     for (int c = 0; c < (PVV ? VE : 1); ++c) accv[h][c] = 0.0f;
-  // PVV: the wave's weights, [tile][token][head] fp32, after its K staging rows
-  float* s_pw = nullptr;
-  if constexpr (PVV) s_pw = reinterpret_cast<float*>(s_kstage + nw * F::KSTAGE) + w * (U * 16 * HG);
 
   // Buffer descriptors end at the split's last token, so rows past it read
   // as zeros (their scores are masked); offsets are 32-bit from the row block.
@@ -886,22 +955,31 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
   struct TileSrc {
     rsrc_t k, v, ks, vs;
     uint32_t off, soff;
+    int pid, in;  // AHEAD: the tile's page and place in it
     bool ok;
   };
-  auto tile_src = [&](int tb) -> TileSrc {
+  // paged: the page of the tile at token tb (-1 past the row's end)
+  auto page_of = [&](int tb) {
+    return tb < hi ? p.page_table[(size_t)b * p.max_pages + (tb >> p.page_log2)] : -1;
+  };
+  auto tile_src = [&](int tb, int pid) -> TileSrc {
     TileSrc t;
     if constexpr (PAGED) {
-      const int pg = tb >> p.page_log2;
-      const int pid = (tb < hi) ? p.page_table[(size_t)b * p.max_pages + pg] : -1;
       t.ok = pid >= 0 && pid < p.num_pages;
-      const int in = tb - (pg << p.page_log2);
+      const int in = tb & ((1 << p.page_log2) - 1);
+      t.pid = pid;
+      t.in = in;
       const uint32_t nrow = t.ok ? (uint32_t)min(16, hi - tb) : 0u;
       const size_t kvb = (size_t)(t.ok ? pid : 0) * p.kv_bs + (size_t)in * ts;
-      const size_t scb = (size_t)(t.ok ? pid : 0) * p.sc_bs + (size_t)in * p.sc_ts;
       t.k = make_rsrc(Kr + kvb, nrow * ts);
       t.v = make_rsrc(Vr + kvb, nrow * ts);
-      t.ks = make_rsrc(F::QUANT ? Ksr + scb : nullptr, nrow * sts);
-      t.vs = make_rsrc(F::QUANT ? Vsr + scb : nullptr, nrow * sts);
+      if constexpr (AHEAD) {  // the lanes address their own scales
+        t.ks = t.vs = t.k;
+      } else {
+        const size_t scb = (size_t)(t.ok ? pid : 0) * p.sc_bs + (size_t)in * p.sc_ts;
+        t.ks = make_rsrc(F::QUANT ? Ksr + scb : nullptr, nrow * sts);
+        t.vs = make_rsrc(F::QUANT ? Vsr + scb : nullptr, nrow * sts);
+      }
       t.off = 0;
       t.soff = 0;
     } else {
@@ -926,19 +1004,30 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
   // matrix cores: the packed score layout (lane: column n, score slots k = tokens 4R + k) is
   // operand B of the PV product of tile jl, zero for the group's other tiles,
   // so column n of O^T gathers tile jl's share of head hh.
-  const int step = 16 * nw;
+  const int step = 16 * tn;
   const int slot0 = TPERM ? R : 4 * R;       // token of the lane's score slot 0 in its tile
   const int lane_tok = jl * step + slot0;  // ... from the base of the lane's group of tiles
-  // scales of paged rows come through per-tile descriptors: every tile's are
-  // loaded and the lane's tile is picked afterwards
-  constexpr bool PICK_SC = F::QUANT && PAGED && P > 1;
   // contiguous, 8-byte aligned scale rows: a lane's four scales (tokens 4R ..
   // 4R + 3, a multiple of 4 from lo) are one 8-byte load in passes that lie
   // wholly before hi (past the descriptor's end a load reads zeros dword by
   // dword, so a dword holding a valid and an invalid scale could lose both)
   const bool vec_sc = F::QUANT && !TPERM && !PAGED && sts == 2u && (lo & 3) == 0 &&
                       ((reinterpret_cast<uintptr_t>(Ksr) | reinterpret_cast<uintptr_t>(Vsr)) & 7u) == 0;
-  for (int pb = lo + 16 * w; pb < hi; pb += U * step) {
+  // scales of paged rows come through per-tile descriptors (unless AHEAD):
+  // every tile's are loaded and the lane's tile is picked afterwards
+  constexpr bool PICK_SC = F::QUANT && PAGED && !AHEAD && P > 1;
+  // AHEAD: four scales of a page as one 8-byte load (every term of a lane's address a
+  // multiple of 4 elements from an 8-byte aligned base)
+  const bool vec_pg = F::QUANT && PAGED && AHEAD && p.sc_ts == 1 && ((p.sc_bs | p.sc_hs) & 3) == 0 &&
+                      ((reinterpret_cast<uintptr_t>(p.Ks) | reinterpret_cast<uintptr_t>(p.Vs)) & 7u) == 0;
+  // AHEAD: page ids a pass ahead, a pass's coming while the one before it is
+  // consumed (one-pass waves would only wait for more of them first)
+  int pid[U];
+  if constexpr (PAGED && AHEAD) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) pid[u] = page_of(lo + 16 * tw + u * step);
+  }
+  for (int pb = lo + 16 * tw; pb < hi; pb += U * step) {
     typename F::KT kr[U][F::KL];
     uint32_t vr[U][4][VD];
     // per-token scales (int8 / int4) of the tokens of the lane's score slots k in its tile of group g
@@ -946,7 +1035,13 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
     _Float16 kt[PICK_SC ? U : 1][4], vt[PICK_SC ? U : 1][4];
     TileSrc src[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) src[u] = tile_src(pb + u * step);
+    for (int u = 0; u < U; ++u) src[u] = tile_src(pb + u * step, !PAGED ? 0 : (AHEAD ? pid[u] : page_of(pb + u * step)));
+    if constexpr (PAGED && AHEAD) {
+      if (pb + U * step < hi) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) pid[u] = page_of(pb + (U + u) * step);
+      }
+    }
     const bool full = !PAGED && pb + (U - 1) * step + 16 <= hi;  // every token of the pass is before hi
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -992,7 +1087,7 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
             }
           }
         }
-      } else {
+      } else if constexpr (!AHEAD) {
         constexpr int T = PICK_SC ? U : NG;  // P == 1 otherwise: tile g is group g
 #pragma unroll
         for (int u = 0; u < T; ++u)
@@ -1028,9 +1123,43 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
         load_vchunk<VG::VBYTES, VD, VCP>(src[u].v, voff + (uint32_t)(VDIRECT ? j : 4 * j) * ts + (F::SOFF_TILE ? 0u : src[u].off),
                                          vr[u][j], F::SOFF_TILE ? src[u].off : 0u);
     }
+    if constexpr (F::QUANT && PAGED && AHEAD) {
+      // Each lane addresses the scales of its own tile (a buffer load's
+      // descriptor is the wave's, so one tile's: loading every tile's and
+      // picking takes 8 U two-byte loads a pass, more than K and V together;
+      // ragged fp8 batch of 64, 12000 tokens at most: 96.5 -> 84.5 us). Only
+      // where waves run many passes: it costs a one-pass call 0.4 us. A tile
+      // never crosses its page, so all 16 slots can be read; those past the
+      // row's end, or of a bad page, count as 0.
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const uint32_t pgl = pick<P>(jm, [&](int j) { return (uint32_t)src[g * P + j].pid; });
+        const uint32_t inl = pick<P>(jm, [&](int j) { return (uint32_t)src[g * P + j].in; });
+        const bool okl = pick<P>(jm, [&](int j) { return src[g * P + j].ok ? ~0u : 0u; }) != 0u;
+        const size_t so = (size_t)(okl ? pgl : 0u) * (size_t)p.sc_bs + (size_t)(inl + slot0) * (uint32_t)p.sc_ts;
+        const _Float16* kp = Ksr + so;
+        const _Float16* vp = Vsr + so;
+        if (vec_pg) {  // four consecutive scales, 8-byte aligned
+          const u2_t a = *reinterpret_cast<const u2_t*>(kp);
+          const u2_t c = *reinterpret_cast<const u2_t*>(vp);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const uint32_t ak = a[k / 2], ck = c[k / 2];
+            ks[g][k] = __builtin_bit_cast(_Float16, (uint16_t)(ak >> (16 * (k % 2))));
+            vs[g][k] = __builtin_bit_cast(_Float16, (uint16_t)(ck >> (16 * (k % 2))));
+          }
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            ks[g][k] = kp[(size_t)(TS * k) * (uint32_t)p.sc_ts];
+            vs[g][k] = vp[(size_t)(TS * k) * (uint32_t)p.sc_ts];
+          }
+        }
+      }
+    }
     __builtin_amdgcn_sched_barrier(0);  // keep every load of the pass ahead of its use
     FQKV_STAMP(1);  // every load of the pass issued
-    if constexpr (QPREP && LAZY) {
+    if constexpr (QPREP && LAZYQ) {
       if (!qready) {
         qprep();
         qready = true;
@@ -1063,7 +1192,7 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
     f4_t c4[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if constexpr (F::STAGE_K) F::stage_k(s_kstage + w * F::KSTAGE, lane, kr[u]);
+      if constexpr (F::STAGE_K) F::stage_k(kstage, lane, kr[u]);
       c4[u] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int i = 0; i < F::NKI; ++i) {
@@ -1095,6 +1224,7 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
           bool ok = pb + g * P * step + lane_tok + TS * k < hi;
           if constexpr (PAGED) ok = ok && pick<P>(jm, [&](int j) { return src[g * P + j].ok ? ~0u : 0u; }) != 0u;
           x[g][k] = ok ? x[g][k] : -INFINITY;
+          if constexpr (PAGED && AHEAD && F::QUANT) vs[g][k] = ok ? vs[g][k] : (_Float16)0.0f;
         }
     }
     // the running maximum is the same in every lane of a head, so it joins
@@ -1335,7 +1465,7 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
         if (h < hcnt) {
 #pragma unroll
           for (int c = 0; c < VE; c += 4)
-            *reinterpret_cast<fl4_t*>(&s_o[w][h][VE * n + c]) =
+            *reinterpret_cast<fl4_t*>(o_dst + h * opitch<D>() + VE * n + c) =
                 fl4_t{accv[h][c], accv[h][c + 1], accv[h][c + 2], accv[h][c + 3]};
         }
       }
@@ -1345,17 +1475,80 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
     if constexpr (!PVV) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        float* dst = &s_o[w][n][VE * (4 * R + k)];
+        float* dst = o_dst + n * opitch<D>() + VE * (4 * R + k);
 #pragma unroll
         for (int c = 0; c < VE; c += 4)
           *reinterpret_cast<fl4_t*>(dst + c) = fl4_t{acc[c][k], acc[c + 1][k], acc[c + 2][k], acc[c + 3][k]};
       }
     }
     if (R == 0) {
-      s_m[n][w] = m_run;
-      s_l[n][w] = l_run;
+      m_dst[n * ml] = m_run;
+      l_dst[n * ml] = l_run;
     }
   }
+}
+
+template <int FMT, int D, int HG, bool PAGED, bool PVV = false, bool KEEPV = false, bool SHORT = false,
+          bool LAZY = false>
+__global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialParams p) {
+  using F = Fmt<FMT, D>;
+  __shared__ __attribute__((aligned(16))) float s_o[NW_MAX][HG][opitch<D>()];
+  __shared__ __attribute__((aligned(16))) float s_m[HG][NW_MAX];
+  __shared__ __attribute__((aligned(16))) float s_l[HG][NW_MAX];
+  __shared__ __attribute__((aligned(16))) float s_mw[NW_MAX][64];  // in-kernel split merge
+  __shared__ float s_mr[NW_MAX][65];
+  __shared__ int s_last;
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_kstage[];  // fp16 K staging, F::KSTAGE bytes per wave
+
+  FQKV_STAMP(0);  // start
+  const int lane = threadIdx.x & 63;
+  // wave index as a scalar, so tile loops branch per wave, not per lane
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nw = blockDim.x >> 6;
+  // blockIdx.x = s * nwsg + wsg or wsg * S + s (wsg = r * ngroups + hg),
+  // decomposed with multiply-shift divisions
+  // Every launch constant in one scalar-load round trip: read here, in the
+  // entry block, so the loads leave together (lazily placed, they took four
+  // dependent round trips before the first KV load, and one more before the
+  // epilogue).
+  pin_sgprs<F::QUANT, PAGED>(p);
+  const uint32_t bq = fast_div(blockIdx.x, p.div_blk);
+  const uint32_t br = blockIdx.x - bq * (uint32_t)p.blk_d;
+  uint32_t wsg = p.split_major ? br : bq;
+  const int s = (int)(p.split_major ? bq : br);
+  {
+    // in a block of 2^(hg_k + hg_d) groups, group e 2^hg_d + c becomes row c 2^hg_k + e:
+    // head e of head set c, the set's heads 2^hg_d groups apart (the identity
+    // when hg_k = hg_d = 0; no branch, so the prologue stays one block)
+    const uint32_t k = (uint32_t)p.hg_k, d = (uint32_t)p.hg_d;
+    const uint32_t low = wsg & ((1u << (k + d)) - 1u);
+    wsg = (wsg - low) | ((low & ((1u << d) - 1u)) << k) | (low >> d);
+  }
+  const uint32_t rr = fast_div(wsg, p.div_groups);
+  const int hg = (int)(wsg - rr * (uint32_t)p.ngroups);
+  const int r = (int)rr;
+  // KV row r = (sequence b, KV head h); its tokens sit kv_ts bytes apart
+  const int b = (int)fast_div((uint32_t)r, p.div_hkv);
+  const int h = r - b * p.hkv;
+  int chunk = p.chunk, nr = p.N;
+  if constexpr (PAGED) {
+    nr = max(min(min(p.seq_lens[b], p.N), p.max_pages << p.page_log2), 0);
+    // the sequence's own length in S parts of whole tiles, no shorter than a pass
+    if (p.own_chunk)
+      chunk = max(16 * (int)fast_div((uint32_t)((nr + 15) >> 4) + (uint32_t)p.S - 1u, p.div_S), p.own_chunk);
+  }
+  const int lo = s * chunk;
+  const int hi = min(lo + chunk, nr);
+  const int hbase = hg * HG;
+  const int hcnt = min(HG, p.G - hbase);
+  const size_t qrow0 = (size_t)r * p.G + hbase;
+  float* s_pw = nullptr;
+  if constexpr (PVV)
+    s_pw = reinterpret_cast<float*>(s_kstage + nw * F::KSTAGE) +
+           w * (tiles_per_pass<FMT, D, HG, false, true>() * 16 * HG);
+  stream_rows<FMT, D, HG, PAGED, PVV, KEEPV, SHORT, LAZY>(p, lane, w, nw, b, h, qrow0, hcnt, lo, hi, &s_o[w][0][0],
+                                                          &s_m[0][w], &s_l[0][w], NW_MAX,
+                                                          kstage_of<F>(s_kstage, w), s_pw);
   FQKV_STAMP(4);  // wave totals written to LDS
   __syncthreads();
   FQKV_STAMP(5);  // wave-merge barrier passed
@@ -1397,9 +1590,11 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
     FQKV_STAMP(7);  // arrival known
     if (s_last) {
       if (p.xcd_local)
-        merge_splits<D, CPOL_SC0>(p.m_part, p.l_part, p.o_part, p.o, qrow0, hcnt, p.S, s_mw, s_mr);
+        merge_splits<D, CPOL_SC0>(SplitAddr{p.m_part, p.l_part, p.o_part, qrow0, p.S}, p.o, qrow0, hcnt, p.S, s_mw,
+                                  s_mr);
       else
-        merge_splits<D, CPOL_SC1>(p.m_part, p.l_part, p.o_part, p.o, qrow0, hcnt, p.S, s_mw, s_mr);
+        merge_splits<D, CPOL_SC1>(SplitAddr{p.m_part, p.l_part, p.o_part, qrow0, p.S}, p.o, qrow0, hcnt, p.S, s_mw,
+                                  s_mr);
       FQKV_STAMP(9);  // merge done
       // every workgroup of the group has counted in: reset for the next call
       if (threadIdx.x == 0) {
@@ -1413,6 +1608,484 @@ __global__ void __launch_bounds__(64 * NW_MAX) decode_partial_kernel(PartialPara
   FQKV_STAMP(10);  // end
 }
 
+// ---- work-balanced decode ----
+//
+// Ragged batches: one workgroup per (row, split) leaves the GPU to the
+// longest row. Here the tiles of all work rows form one line that the waves
+// of the resident workgroups cut into equal spans (a workgroup's waves take
+// neighbouring ones). A wave streams its span row by row on its own; a row it
+// holds whole it emits at once, and of the first and last row of its span it
+// may hold a piece. The pieces meet in LDS once the workgroup's waves are
+// through: rows that end there are emitted, and the workgroup's own first and
+// last piece go to scratch, where the last workgroup to finish a row's pieces
+// merges them, as in the split merge. Nobody waits on another workgroup.
+// Bound by HBM once the waves stream; what is left is the longest wave of a
+// CU (a SIMD's older waves are served first) and ~6 us of fixed cost (lengths
+// and place 1.5 us, the last pieces' merge 3-4 us). Against one workgroup per
+// (row, split), 32 query / 8 KV heads, D 128: fp16, 32 sequences of 120 to
+// 7700 tokens 107.5 -> 49.7 us (2.3 -> 5.0 TB/s); fp8, 64 sequences of 300 to
+// 12000 tokens 199 -> 84.5 us (2.1 -> 5.1 TB/s). Tiles of a workgroup dealt
+// to its waves in turn (every wave then starts and ends every row) measured
+// 62 and 116 us; more workgroups than are resident 55-65 and 94-109 us.
+
+// Inclusive prefix sum over the wave's lanes (DPP row_shr within the 16-lane
+// rows, then the row totals).
+__device__ __forceinline__ uint32_t wave_scan(uint32_t x, int lane) {
+  x += (uint32_t)dpp_i<0x111>((int)x);
+  x += (uint32_t)dpp_i<0x112>((int)x);
+  x += (uint32_t)dpp_i<0x114>((int)x);
+  x += (uint32_t)dpp_i<0x118>((int)x);
+  const uint32_t r0 = __builtin_amdgcn_readlane(x, 15), r1 = __builtin_amdgcn_readlane(x, 31),
+                 r2 = __builtin_amdgcn_readlane(x, 47);
+  // masks instead of selects, which the compiler turned into branches
+  const uint32_t m1 = (uint32_t)((15 - lane) >> 31), m2 = (uint32_t)((31 - lane) >> 31),
+                 m3 = (uint32_t)((47 - lane) >> 31);
+  return x + (r0 & m1) + (r1 & m2) + (r2 & m3);
+}
+
+// Maximum over the wave of non-negative values.
+__device__ __forceinline__ int wave_max_i(int k) {
+  k = max(k, dpp_i<0xB1>(k));
+  k = max(k, dpp_i<0x4E>(k));
+  k = max(k, dpp_i<0x141>(k));
+  k = max(k, dpp_i<0x140>(k));
+  return __builtin_amdgcn_readfirstlane(rows4_max_key(k));
+}
+
+// x / d for a quotient below 2^22 and x below 2^31, wave-uniform: the fp32
+// estimate is off by at most one.
+__device__ __forceinline__ uint32_t small_div(uint32_t x, uint32_t d) {
+  uint32_t q = (uint32_t)((float)x * __builtin_amdgcn_rcpf((float)d));
+  int r = (int)(x - q * d);
+  q = r < 0 ? q - 1u : (r >= (int)d ? q + 1u : q);
+  return __builtin_amdgcn_readfirstlane(q);
+}
+
+// The line of work. A row takes row_cost units (what starting it costs a
+// wave) and one per tile; an empty sequence has one tile, so it is somebody's
+// work and gets its zeros. Each wave adds up the sequences' units itself, 256
+// sequences at a time, four to a lane.
+typedef int i4_t __attribute__((ext_vector_type(4)));
+struct WorkLine {
+  const int* seq_lens;
+  int nb, most, row_cost;  // sequences, most tokens of one
+  int lane;
+  i4_t n0;               // tokens of sequences 4 lane ..
+  uint32_t sum0, scan0;  // units of their rows, prefix sum up to and with them
+  uint32_t total;        // units of all rows of a plane
+  uint32_t wgs;          // workgroups that get a span
+  uint32_t span, longer;  // units per workgroup; the first `longer` take one more
+
+  __device__ __forceinline__ static uint32_t tiles(int n) { return n > 16 ? (uint32_t)(n + 15) >> 4 : 1u; }
+  __device__ __forceinline__ uint32_t units(int n) const { return tiles(n) + (uint32_t)row_cost; }
+  // sequences b0 + 4 lane ..: tokens, sum and scan of units
+  __device__ __forceinline__ void load4(int b0, i4_t& n, uint32_t& sum, uint32_t& scan) const {
+    // (zeros past the last sequence, whose units are masked: no branches)
+    const rsrc_t r = make_rsrc(seq_lens, (uint32_t)nb * 4u);
+    const int b = b0 + 4 * lane;
+    uint32_t v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = buf_load<4>(r, (uint32_t)(b + k) * 4u);
+    sum = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int nk = min((int)v[k], most);
+      sum += units(nk) & (uint32_t)((b + k - nb) >> 31);
+      n[k] = nk;
+    }
+    scan = wave_scan(sum, lane);
+  }
+  // tokens of sequence b (wave-uniform)
+  __device__ __forceinline__ int tokens(int b) const {
+    if (b >= 256) return min(seq_lens[b], most);
+    const int l = b >> 2;
+    const int a = (b & 1) ? n0.y : n0.x, c = (b & 1) ? n0.w : n0.z;
+    return __builtin_amdgcn_readlane((b & 2) ? c : a, l);
+  }
+
+  __device__ __forceinline__ WorkLine(const BalancedParams& p, int lane_)
+      : seq_lens(p.seq_lens),
+        nb(p.nb),
+        most(min(p.N, p.max_pages << p.page_log2)),
+        row_cost(p.row_cost),
+        lane(lane_) {
+    load4(0, n0, sum0, scan0);
+    uint32_t seqs = __builtin_amdgcn_readlane(scan0, 63);
+    int longest = max(max(n0.x, n0.y), max(n0.z, n0.w));
+    for (int b0 = 256; b0 < p.nb; b0 += 256) {
+      i4_t n;
+      uint32_t sum, scan;
+      load4(b0, n, sum, scan);
+      seqs += __builtin_amdgcn_readlane(scan, 63);
+      longest = max(longest, max(max(n.x, n.y), max(n.z, n.w)));
+    }
+    total = seqs * (uint32_t)p.rg;
+    // Spans equal to within a unit, for every workgroup of the launch. But a
+    // short line gets spans no shorter than min_span or (if that is less) the
+    // average row, and sequences of one length (in tiles) get the number of
+    // spans that cuts every row alike, if that leaves few workgroups out
+    // (p.aligned): no row then starts or ends inside a span.
+    const uint32_t least = min((uint32_t)p.min_span, fast_div(total, p.div_rows));
+    wgs = (uint32_t)p.nspan;
+    span = fast_div(total, p.div_nspan);
+    if (span < least) {
+      wgs = small_div(total + least - 1u, least);
+      span = small_div(total, wgs);
+    } else if (p.aligned && units(wave_max_i(longest)) * (uint32_t)nb == seqs) {
+      wgs = (uint32_t)p.aligned;
+      span = fast_div(total, p.div_aligned);
+    }
+    longer = total - span * wgs;
+  }
+  __device__ __forceinline__ uint32_t wg_start(uint32_t i) const { return i * span + min(i, longer); }
+  // the workgroup that holds unit x
+  __device__ __forceinline__ uint32_t wg_of(uint32_t x) const {
+    const uint32_t cut = longer * (span + 1u);
+    const bool lo = x < cut;
+    return (lo ? 0u : longer) + small_div(lo ? x : x - cut, lo ? span + 1u : span);
+  }
+  // first workgroup and number of workgroups of units x .. x + n - 1
+  __device__ __forceinline__ void wgs_of(uint32_t x, uint32_t n, uint32_t& first, int& count) const {
+    first = wg_of(x);
+    count = (int)(wg_of(x + n - 1u) - first) + 1;
+  }
+  // f(first sequence of the lane's four, n, sum, scan, units before the block)
+  // on the block of 256 sequences for which pick(...) holds, the last at the latest
+  template <typename Pick, typename F>
+  __device__ __forceinline__ void in_block(Pick pick, F f) const {
+    uint32_t base = 0;
+    i4_t n = n0;
+    uint32_t sum = sum0, scan = scan0;
+    for (int b0 = 0;;) {
+      const uint32_t end = base + __builtin_amdgcn_readlane(scan, 63);
+      if (pick(b0, end) || b0 + 256 >= nb) {
+        f(b0, n, sum, scan, base);
+        return;
+      }
+      base = end;
+      b0 += 256;
+      load4(b0, n, sum, scan);
+    }
+  }
+  // the sequence that holds unit u of the line of one row per sequence, the
+  // units of its row and the units before it (all wave-uniform)
+  __device__ __forceinline__ void find(uint32_t u, int& b, uint32_t& ub, uint32_t& before) const {
+    in_block([&](int, uint32_t end) { return u < end; },
+             [&](int b0, i4_t n, uint32_t sum, uint32_t scan, uint32_t base) {
+               const uint64_t m = __builtin_amdgcn_ballot_w64(base + scan > u);
+               const int l = m ? __builtin_ctzll(m) : 63;
+               b = b0 + 4 * l;
+               before = base + __builtin_amdgcn_readlane(scan, l) - __builtin_amdgcn_readlane(sum, l);
+               ub = units(__builtin_amdgcn_readlane(n[0], l));
+#pragma unroll
+               for (int k = 1; k < 4; ++k) {
+                 const bool next = u >= before + ub && b + 1 < nb;
+                 before += next ? ub : 0u;
+                 b += next;
+                 ub = next ? units(__builtin_amdgcn_readlane(n[k], l)) : ub;
+               }
+             });
+  }
+  // units before sequence bq
+  __device__ __forceinline__ uint32_t before(int bq) const {
+    uint32_t r = 0;
+    in_block([&](int b0, uint32_t) { return bq < b0 + 256; },
+             [&](int b0, i4_t n, uint32_t sum, uint32_t scan, uint32_t base) {
+               const int l = (bq - b0) >> 2;
+               r = base + __builtin_amdgcn_readlane(scan, l) - __builtin_amdgcn_readlane(sum, l);
+#pragma unroll
+               for (int k = 0; k < 3; ++k)
+                 r += b0 + 4 * l + k < bq ? units(__builtin_amdgcn_readlane(n[k], l)) : 0u;
+             });
+    return r;
+  }
+};
+
+template <int FMT, int D, int HG>
+__global__ void __launch_bounds__(64 * balanced_nw(FMT, D, HG), balanced_waves(FMT, D, HG))
+    decode_balanced_kernel(BalancedParams p) {
+  using F = Fmt<FMT, D>;
+  constexpr int NWM = balanced_nw(FMT, D, HG);
+  // per wave: region 0 keeps the piece of a row begun by another wave, region
+  // 1 rows and pieces begun here (and, while streaming, the K staging rows)
+  constexpr int REG = HG * opitch<D>() * 4;
+  constexpr int REG1 = F::STAGE_K && kstage_bytes<F>() > REG ? kstage_bytes<F>() : REG;
+  __shared__ __attribute__((aligned(16))) uint8_t s_buf[NWM][REG + REG1];
+  __shared__ __attribute__((aligned(16))) float s_m[2][HG][NWM], s_l[2][HG][NWM];
+  __shared__ __attribute__((aligned(16))) float s_mw[NWM][64];
+  __shared__ float s_mr[NWM][65];
+  // The rows of the waves' pieces, four words each: where the row ends on the
+  // line, first query head, work row, and first workgroup that holds it (13
+  // bits), workgroups (13), query heads (0: no piece). Wave w's region r is
+  // record 2w + r, so a wave reads all of them with one load.
+  static_assert(NWM <= 8, "one word of the piece records per lane");
+  __shared__ uint32_t s_rec[64];
+  __shared__ uint32_t s_start[NWM];
+  __shared__ int s_last[2];
+
+  FQKV_STAMP(0);
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t nw = blockDim.x >> 6;
+  auto region = [&](int w_, int r) { return reinterpret_cast<float*>(&s_buf[w_][r ? REG : 0]); };
+  const WorkLine line(p, lane);
+  // Workgroup i of head e of every head set. Workgroups are dealt to the
+  // XCDs in turn by blockIdx.x; each XCD gets `per` neighbouring spans, so the
+  // pieces of most rows meet in one L2, and the heads of a set run on one XCD.
+  const uint32_t per = (line.wgs + 7u) >> 3;
+  const uint32_t xcd = blockIdx.x & 7u;
+  const uint32_t q0 = blockIdx.x >> 3;
+  const uint32_t e = q0 & ((1u << p.hk) - 1u);
+  if ((q0 >> p.hk) >= per) return;  // the whole workgroup
+  const uint32_t i = xcd * per + (q0 >> p.hk);
+  // a row's pieces all come from this XCD, whose L2 then serves as in the
+  // XCD-local split merge (the flag is the host's: the probe, the CU mask)
+  auto xcd_local = [&](uint32_t first, int count) {
+    return p.xcd_local && first >= xcd * per && first + (uint32_t)count <= (xcd + 1u) * per;
+  };
+  // the wave's first row: sequence b (U units a row), row `in` of the
+  // sequence, its unit y; t .. t1 - 1 the wave's span, wg0 .. wg1 - 1 the
+  // workgroup's; rs the row's place on the line
+  const uint32_t rc = (uint32_t)p.row_cost;
+  int b = 0;
+  uint32_t U = 1, in = 0, y = 0, t, t1, rs = 0, wg0, wg1;
+  wg0 = __builtin_amdgcn_readfirstlane(line.wg_start(i));
+  const uint32_t total = __builtin_amdgcn_readfirstlane(line.total);
+  if (wg0 >= total) return;  // the whole workgroup
+  wg1 = min((uint32_t)__builtin_amdgcn_readfirstlane(line.wg_start(i + 1u)), total);
+  const uint32_t wgn = wg1 - wg0;
+  const uint32_t lw = 31u - (uint32_t)__builtin_clz(nw);  // 2, 4 or 8 waves
+  t = wg0 + (wgn * (uint32_t)w >> lw);
+  t1 = wg0 + (wgn * (uint32_t)(w + 1) >> lw);
+  if (lane == 0) s_start[w] = t;
+  if (t < t1) {
+    uint32_t before;
+    line.find(fast_div(t, p.div_rg), b, U, before);
+    const uint32_t x = t - before * (uint32_t)p.rg;
+    in = small_div(x, U);
+    y = x - in * U;
+    rs = t - y;
+  }
+  if (lane < 8) s_rec[8 * w + lane] = 0;
+  FQKV_STAMP(2);  // the wave's place on the line known
+  while (t < t1) {
+    const uint32_t n = min(U - y, t1 - t);  // units of the row in this span
+    const uint32_t T = U - rc;
+    const uint32_t ta = y > rc ? y - rc : 0u, tb = y + n > rc ? y + n - rc : 0u;  // its tiles
+    if (ta < tb) {
+      // KV head and query-head group of the work row
+      const int hs = (int)fast_div(in, p.div_groups);
+      const int hg = (int)in - hs * p.ngroups;
+      const int h = (hs << p.hk) + (int)e;
+      const int hcnt = min(HG, p.G - hg * HG);
+      const size_t row = (size_t)b * p.hkv + h;
+      const size_t qrow0 = row * p.G + hg * HG;
+      const int kind = ta == 0 ? 1 : 0;
+      stream_rows<FMT, D, HG, true, false, false, false, false, true>(
+          p, lane, 0, 1, b, h, qrow0, hcnt, (int)ta * 16, min((int)tb * 16, line.tokens(b)), region(w, kind),
+          &s_m[kind][0][w], &s_l[kind][0][w], NWM, &s_buf[w][REG], nullptr);
+      if (tb - ta == T) {  // whole: the wave's own LDS rows, in order
+        const float* so = region(w, 1);
+        for (int idx = 4 * lane; idx < hcnt * D; idx += 256) {
+          const int hh = idx / D;
+          const int d = idx - hh * D;
+          put_output(p.o + (qrow0 + hh) * D + d, s_l[1][hh][w],
+                     *reinterpret_cast<const fl4_t*>(so + hh * opitch<D>() + d));
+        }
+      } else {
+        uint32_t first;
+        int count;
+        line.wgs_of(rs + rc, T, first, count);
+        if (lane == 0) {
+          uint32_t* rec = s_rec + 8 * w + 4 * kind;
+          rec[0] = rs + U;
+          rec[1] = (uint32_t)qrow0;
+          rec[2] = (uint32_t)(row * p.ngroups) + (uint32_t)hg;
+          rec[3] = first | (uint32_t)count << 13 | (uint32_t)hcnt << 26;
+        }
+      }
+    }
+    t += n;
+    y = 0;
+    rs += U;
+    if (++in == (uint32_t)p.rg && t < t1) {
+      in = 0;
+      ++b;
+      U = line.units(line.tokens(b));
+    }
+  }
+  FQKV_STAMP(4);  // the wave's span streamed
+  __syncthreads();
+  FQKV_STAMP(5);
+  // Rows in pieces, by the piece that comes first in the workgroup: the first
+  // wave's region 0 or any wave's region 1; the waves after it hold theirs in
+  // region 0. At most the first and the last row leave the workgroup unfinished.
+  // (In a span shorter than the waves are many, some waves have no part; the
+  // wave that has unit x is the last one that starts at or before it.)
+  const uint32_t rec = lane < 8 * (int)nw ? s_rec[lane] : 0u;
+  const uint32_t start = lane < (int)nw ? s_start[lane] : ~0u;
+  auto wave_of = [&](uint32_t x) { return 63 - __builtin_clzll(__builtin_amdgcn_ballot_w64(start <= x)); };
+  struct PieceRow {
+    uint32_t end;
+    int qrow0, hcnt, group;
+    uint32_t first;
+    int count;
+  };
+  PieceRow out[2] = {{0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0}};
+  const uint64_t pieces = __builtin_amdgcn_ballot_w64((lane & 3) == 3 && rec >> 26 != 0);  // bit 8w + 4r + 3
+  uint64_t rows = pieces & (0x8080808080808080ull | 8ull << 8 * wave_of(wg0));
+  while (rows) {
+    const int j = __builtin_ctzll(rows);
+    rows &= rows - 1;
+    const int k = j >> 3, kind = j >> 2 & 1;
+    const uint32_t packed = __builtin_amdgcn_readlane(rec, j);
+    PieceRow r;
+    r.end = __builtin_amdgcn_readlane(rec, j - 3);
+    r.qrow0 = (int)__builtin_amdgcn_readlane(rec, j - 2);
+    r.group = (int)__builtin_amdgcn_readlane(rec, j - 1);
+    r.first = packed & 8191u;
+    r.count = (int)(packed >> 13 & 8191u);
+    r.hcnt = (int)(packed >> 26);
+    const int last = wave_of(min(r.end, wg1) - 1u);  // waves k .. last hold it
+    const bool whole = r.count == 1;
+    // region 0 of waves k + 1 .. last, bit 8w + 3
+    const uint64_t others = pieces & 0x0808080808080808ull & ((2ull << (8 * last + 6)) - (1ull << (8 * k + 7)));
+    const bool local = xcd_local(r.first, r.count);
+    const size_t entry = 2 * ((size_t)e * p.nspan + i) + kind;
+    for (int idx = 4 * (int)threadIdx.x; idx < r.hcnt * D; idx += 4 * (int)blockDim.x) {
+      const int hh = idx / D;
+      const int d = idx - hh * D;
+      // every wave's (m, l) and acc read (those that hold no part of the row
+      // weigh nothing), all reads in flight together
+      float mw[NWM], lw_[NWM];
+      fl4_t a[NWM];
+      lds_row<NWM>(s_m[0][hh], mw);
+      lds_row<NWM>(s_l[0][hh], lw_);
+      const float mk = s_m[kind][hh][k], lk = s_l[kind][hh][k];
+#pragma unroll
+      for (int q = 0; q < NWM; ++q)
+        a[q] = *reinterpret_cast<const fl4_t*>(region(others >> (8 * q + 3) & 1 ? q : k, others >> (8 * q + 3) & 1 ? 0 : kind) +
+                                               hh * opitch<D>() + d);
+      __builtin_amdgcn_sched_barrier(0);
+      float M = mk;
+#pragma unroll
+      for (int q = 0; q < NWM; ++q) {
+        const bool other = others >> (8 * q + 3) & 1;  // wave-uniform
+        mw[q] = q == k ? mk : (other ? mw[q] : -INFINITY);
+        lw_[q] = q == k ? lk : (other ? lw_[q] : 0.0f);
+        M = fmaxf(M, mw[q]);
+      }
+      const float Mu = (M == -INFINITY) ? 0.0f : M;
+      float L = 0.0f;
+      fl4_t O = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int q = 0; q < NWM; ++q) {
+        if (q == k || (others >> (8 * q + 3) & 1)) {
+          const float wq = fast_exp2((mw[q] - Mu) * p.c);
+          L = fmaf(wq, lw_[q], L);
+          O.x = fmaf(wq, a[q].x, O.x);
+          O.y = fmaf(wq, a[q].y, O.y);
+          O.z = fmaf(wq, a[q].z, O.z);
+          O.w = fmaf(wq, a[q].w, O.w);
+        }
+      }
+      if (whole) {
+        put_output(p.o + (size_t)(r.qrow0 + hh) * D + d, L, O);
+      } else {  // read by another workgroup of this launch, on this XCD or on any
+        float* pe = p.m_part + entry * entry_floats(D, HG);
+        const rsrc_t rP = make_rsrc(pe + 32, (uint32_t)(HG * D) * 4u);
+        const u4_t bits = __builtin_bit_cast(u4_t, O);
+        const float mo = (M == -INFINITY) ? -INFINITY : M * p.scale;
+        if (local) {
+          if (d == 0) {
+            __hip_atomic_store(pe + hh, mo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_store(pe + 16 + hh, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          }
+          __builtin_amdgcn_raw_buffer_store_b128(bits, rP, (hh * D + d) * 4, 0, CPOL_SC0);
+        } else {
+          if (d == 0) {
+            __hip_atomic_store(pe + hh, mo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(pe + 16 + hh, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+          __builtin_amdgcn_raw_buffer_store_b128(bits, rP, (hh * D + d) * 4, 0, CPOL_SC1);
+        }
+      }
+    }
+    if (!whole) {
+      if (kind)
+        out[1] = r;
+      else
+        out[0] = r;
+    }
+  }
+  FQKV_STAMP(6);  // outputs and pieces issued
+  const bool have0 = out[0].hcnt != 0, have1 = out[1].hcnt != 0;
+  if (p.slot < 0 || !(have0 || have1)) return;
+  // every piece stored and acknowledged, then counted in; the last of a row's
+  // workgroups merges it (see the split merge of decode_partial_kernel)
+  const bool local0 = xcd_local(out[0].first, out[0].count), local1 = xcd_local(out[1].first, out[1].count);
+  int* ctr0 = arrival_counter(p.slot, (uint32_t)out[0].group);
+  int* ctr1 = arrival_counter(p.slot, (uint32_t)out[1].group);
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    const bool second = threadIdx.x == 1;
+    int* ctr = second ? ctr1 : ctr0;
+    int before = -1;
+    if (second ? have1 : have0)
+      before = (second ? local1 : local0)
+                   ? __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
+                   : __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last[threadIdx.x] = before >= 0 && before == (second ? out[1].count : out[0].count) - 1;
+  }
+  __syncthreads();
+  FQKV_STAMP(7);  // arrivals known
+  const bool last0 = s_last[0] != 0, last1 = s_last[1] != 0;
+#pragma unroll 1
+  for (int j = last0 ? 0 : 1; j < (last1 ? 2 : 1); ++j) {
+    const size_t entry = 2 * ((size_t)e * p.nspan + (j ? out[1].first : out[0].first)) + 1;
+    const PieceAddr<D, HG> ad{p.m_part + entry * entry_floats(D, HG)};
+    const size_t qrow0 = (size_t)(j ? out[1].qrow0 : out[0].qrow0);
+    const int hcnt = j ? out[1].hcnt : out[0].hcnt, count = j ? out[1].count : out[0].count;
+    // every piece of the row is counted in: reset for the next call
+    if (j ? local1 : local0) {
+      merge_splits<D, CPOL_SC0>(ad, p.o, qrow0, hcnt, count, s_mw, s_mr);
+      if (threadIdx.x == 0)
+        __hip_atomic_store(j ? ctr1 : ctr0, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    } else {
+      merge_splits<D, CPOL_SC1>(ad, p.o, qrow0, hcnt, count, s_mw, s_mr);
+      if (threadIdx.x == 0)
+        __hip_atomic_store(j ? ctr1 : ctr0, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();  // the merge's LDS rows serve both rows
+  }
+  FQKV_STAMP(10);
+}
+
+// The pieces of every row merged by a second kernel, one workgroup per work
+// row (calls without an arrival-counter slot).
+template <int D, int HG>
+__global__ void __launch_bounds__(256) combine_pieces_kernel(BalancedParams p) {
+  __shared__ __attribute__((aligned(16))) float s_w[4][64];
+  __shared__ float s_red[4][65];
+  const int lane = threadIdx.x & 63;
+  const WorkLine line(p, lane);
+  const uint32_t e = blockIdx.x & ((1u << p.hk) - 1u), i = blockIdx.x >> p.hk;
+  const int b = (int)fast_div(i, p.div_rg);
+  const uint32_t in = i - (uint32_t)b * (uint32_t)p.rg;
+  const uint32_t U = line.units(line.tokens(b)), rc = (uint32_t)p.row_cost;
+  uint32_t first;
+  int count;
+  line.wgs_of(line.before(b) * (uint32_t)p.rg + in * U + rc, U - rc, first, count);
+  if (count < 2) return;  // emitted whole
+  const int hs = (int)fast_div(in, p.div_groups);
+  const int hg = (int)in - hs * p.ngroups;
+  const size_t row = (size_t)b * p.hkv + (hs << p.hk) + (int)e;
+  const size_t entry = 2 * ((size_t)e * p.nspan + first) + 1;
+  const PieceAddr<D, HG> ad{p.m_part + entry * entry_floats(D, HG)};
+  merge_splits<D, 0>(ad, p.o, row * p.G + hg * HG, min(HG, p.G - hg * HG), count, s_w, s_red);
+}
+
 // Two-kernel form of the split merge (decode_attn_gqa_sk_fast.cu:57-94): one
 // workgroup per query head. Used when a call cannot take arrival counters.
 template <int D>
@@ -1422,7 +2095,7 @@ __global__ void __launch_bounds__(64 * NW_MAX) combine_kernel(const float* __res
                                                               _Float16* __restrict__ o, int S) {
   __shared__ __attribute__((aligned(16))) float s_w[NW_MAX][64];
   __shared__ float s_red[NW_MAX][65];
-  merge_splits<D, 0>(m_part, l_part, o_part, o, blockIdx.x, 1, S, s_w, s_red);
+  merge_splits<D, 0>(SplitAddr{m_part, l_part, o_part, blockIdx.x, S}, o, blockIdx.x, 1, S, s_w, s_red);
 }
 
 // Dequantise through the kernels' own conversions (K side: int -> fp16
@@ -1554,17 +2227,22 @@ static std::atomic<int> g_pv_valu{0};
 void set_pv_valu(int on) { g_pv_valu.store(on ? 1 : 0, std::memory_order_relaxed); }
 
 template <int FMT, int D, int HG>
-static hipError_t launch_partial_t(const PartialParams& p, int nblocks, int nw, hipStream_t st) {
+static hipError_t launch_partial_t(const PartialParams& params, int nblocks, int nw, hipStream_t st) {
   // nw is a maximum: a split shorter than one pass of nw waves would leave
   // waves with nothing to load, so take the fewest waves (at least 2) that
   // still cover the split in one pass -- but, when the splits are merged in
   // the kernel, no fewer than the merge has (head, 64-dim block) units, so
   // that every unit keeps a wave of its own.
   {
-    const int u = p.page_table ? tiles_per_pass<FMT, D, HG, true, false>() : tiles_per_pass<FMT, D, HG, false, false>();
-    const int tiles = (p.chunk + 15) / 16;
-    const int units = p.S > 1 ? HG * (D / 64) : 1;
+    const int u = params.page_table ? tiles_per_pass<FMT, D, HG, true, false>() : tiles_per_pass<FMT, D, HG, false, false>();
+    const int tiles = (params.chunk + 15) / 16;
+    const int units = params.S > 1 ? HG * (D / 64) : 1;
     while (nw > 2 && nw / 2 >= units && (nw / 2) * u >= tiles) nw /= 2;
+  }
+  PartialParams p = params;
+  if (p.own_chunk) {  // a pass of the workgroup, if a split is longer
+    p.own_chunk = 16 * nw * tiles_per_pass<FMT, D, HG, true, false>();
+    if (p.chunk <= p.own_chunk) p.own_chunk = 0;
   }
   size_t lds = 0;
   if constexpr (Fmt<FMT, D>::STAGE_K) lds = (size_t)nw * Fmt<FMT, D>::KSTAGE;
@@ -1656,6 +2334,7 @@ hipError_t launch_partial(int fmt, int D, int hg, const PartialParams& params, i
   p.div_blk = make_fastdiv((uint32_t)p.blk_d);
   p.div_groups = make_fastdiv((uint32_t)p.ngroups);
   p.div_hkv = make_fastdiv((uint32_t)p.hkv);
+  p.div_S = make_fastdiv((uint32_t)p.S);
   switch (fmt) {
     case KV_F16: return D == 64 ? launch_partial_d<KV_F16, 64>(hg, p, nblocks, nw, st)
                                 : launch_partial_d<KV_F16, 128>(hg, p, nblocks, nw, st);
@@ -1667,6 +2346,62 @@ hipError_t launch_partial(int fmt, int D, int hg, const PartialParams& params, i
                                  : launch_partial_d<KV_BF16, 128>(hg, p, nblocks, nw, st);
     case KV_FP8: return D == 64 ? launch_partial_d<KV_FP8, 64>(hg, p, nblocks, nw, st)
                                 : launch_partial_d<KV_FP8, 128>(hg, p, nblocks, nw, st);
+  }
+  return hipErrorInvalidValue;
+}
+
+template <int FMT, int D, int HG>
+static hipError_t launch_balanced_t(const BalancedParams& p, int nw, hipStream_t st) {
+  if (nw > balanced_nw(FMT, D, HG)) return hipErrorInvalidValue;
+  const unsigned rows = (unsigned)(p.nb * p.rg) << p.hk;
+  const unsigned grid = (unsigned)p.nspan << p.hk;
+  hipLaunchKernelGGL((decode_balanced_kernel<FMT, D, HG>), dim3(grid), dim3(64 * nw), 0, st, p);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess && p.slot < 0) {
+    hipLaunchKernelGGL((combine_pieces_kernel<D, HG>), dim3(rows), dim3(256), 0, st, p);
+    e = hipGetLastError();
+  }
+  return e;
+}
+template <int FMT, int D>
+static hipError_t launch_balanced_d(int hg, const BalancedParams& p, int nw, hipStream_t st) {
+  switch (hg) {
+    case 1: return launch_balanced_t<FMT, D, 1>(p, nw, st);
+    case 2: return launch_balanced_t<FMT, D, 2>(p, nw, st);
+    case 4: return launch_balanced_t<FMT, D, 4>(p, nw, st);
+    case 8: return launch_balanced_t<FMT, D, 8>(p, nw, st);
+    case 16: return launch_balanced_t<FMT, D, 16>(p, nw, st);
+  }
+  return hipErrorInvalidValue;
+}
+hipError_t launch_balanced(int fmt, int D, int hg, const BalancedParams& params, int nw, hipStream_t st,
+                           int* xcd_local) {
+  if ((nw != 2 && nw != 4 && nw != 8) || params.nb < 1 || params.nb > BALANCED_MAX_SEQS || params.rg < 1 ||
+      params.nspan < 8 || params.nspan > BALANCED_MAX_SPANS || params.nspan % 8 || params.hk < 0 || !params.page_table ||
+      !params.m_part || params.min_span < 1)
+    return hipErrorInvalidValue;
+  BalancedParams p = params;
+  p.div_groups = make_fastdiv((uint32_t)p.ngroups);
+  p.div_hkv = make_fastdiv((uint32_t)p.hkv);
+  p.div_rg = make_fastdiv((uint32_t)p.rg);
+  p.div_rows = make_fastdiv((uint32_t)p.nb * (uint32_t)p.rg);
+  // (no more rows than counter lines: rows that share one may meet on different XCDs)
+  p.xcd_local = p.slot >= 0 && p.xcd_ok && ((int64_t)p.nb * p.rg << p.hk) <= ARRIVAL_LINES &&
+                xcd_period(st) == 8;
+  if (xcd_local) *xcd_local = p.xcd_local;
+  // all rows cut alike by k spans each, if 7/8 of the workgroups get one
+  const int nrows = p.nb * p.rg;
+  p.aligned = p.nspan / nrows * nrows;
+  if (p.aligned * 8 < p.nspan * 7) p.aligned = 0;
+  p.div_aligned = make_fastdiv((uint32_t)(p.aligned ? p.aligned : 1));
+  p.div_nspan = make_fastdiv((uint32_t)p.nspan);
+  p.div_blk = p.div_hkv;  // unused: the kernel has no split decomposition
+  switch (fmt) {
+    case KV_F16: return D == 64 ? launch_balanced_d<KV_F16, 64>(hg, p, nw, st) : launch_balanced_d<KV_F16, 128>(hg, p, nw, st);
+    case KV_I8: return D == 64 ? launch_balanced_d<KV_I8, 64>(hg, p, nw, st) : launch_balanced_d<KV_I8, 128>(hg, p, nw, st);
+    case KV_I4: return D == 64 ? launch_balanced_d<KV_I4, 64>(hg, p, nw, st) : launch_balanced_d<KV_I4, 128>(hg, p, nw, st);
+    case KV_BF16: return D == 64 ? launch_balanced_d<KV_BF16, 64>(hg, p, nw, st) : launch_balanced_d<KV_BF16, 128>(hg, p, nw, st);
+    case KV_FP8: return D == 64 ? launch_balanced_d<KV_FP8, 64>(hg, p, nw, st) : launch_balanced_d<KV_FP8, 128>(hg, p, nw, st);
   }
   return hipErrorInvalidValue;
 }

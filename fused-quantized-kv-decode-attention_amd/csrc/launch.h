@@ -71,10 +71,13 @@ struct PartialParams {
   int max_pages;
   int page_log2;
   int num_pages;
+  // paged: every sequence in S parts of its own length, no shorter than this
+  // (0: of chunk tokens); the caller sets 1, launch_partial a pass's tokens
+  int own_chunk;
   // set by launch_partial from S, ngroups and hkv
   int split_major;  // blockIdx.x = s * nwsg + wsg (else wsg * S + s)
   int blk_d;        // the divisor of that decomposition: nwsg or S
-  FastDiv div_blk, div_groups, div_hkv;
+  FastDiv div_blk, div_groups, div_hkv, div_S;
   // Head grouping (hg_k = 0: off): in a token-major layout the rows of 2^hg_k
   // neighbouring KV heads share each 128-byte line of a token (two 64-byte
   // int4 rows at D 128). Group wsg is then renumbered so those heads' work
@@ -84,6 +87,30 @@ struct PartialParams {
   // changes, so results do not depend on where workgroups run.
   int hg_k, hg_d;   // log2 heads per span, log2 distance between them in group order
 };
+
+// Work-balanced launch (decode_balanced_kernel). The tiles (16 tokens) of
+// every work row -- (sequence, KV head, query-head group), sequence-major --
+// form one line, cut into equal spans, one per workgroup, whose waves take equal
+// parts; a span may begin and end inside a row. m_part holds two entries of
+// entry_floats(D, hg) floats per workgroup, 128-byte aligned: the pieces of
+// rows it does not finish.
+// hk: the rows of 2^hk neighbouring KV heads share each 128-byte line of a
+// token; the heads of such a set get the same spans on workgroups 8 apart
+// (one XCD), so the line's rows count sets instead of heads.
+struct BalancedParams : PartialParams {
+  int nb;        // sequences
+  int nspan;     // workgroups per head of a set, a multiple of 8
+  int hk;        // log2 heads per set
+  int rg;        // work rows per sequence and head of a set: (hkv >> hk) * ngroups
+  int row_cost;  // units a row takes on the line besides its tiles
+  int min_span;  // least units per workgroup (but no more than a row has on average)
+  // set by launch_balanced
+  int aligned;  // spans that cut every row alike when all rows are as long (0: none)
+  FastDiv div_nspan, div_rg, div_rows, div_aligned;  // by nspan, rg, nb * rg and aligned
+};
+constexpr int entry_floats(int D, int hg) { return 32 + hg * D; }
+constexpr int BALANCED_MAX_SPANS = 8184;  // (13 bits, a multiple of 8)
+constexpr int BALANCED_MAX_SEQS = 4096;  // sequences (every wave adds up their lengths)
 
 // The reference's contiguous layout: K, V [rows, N, row_bytes], scales [rows, N].
 inline void set_contiguous_layout(PartialParams& p, int64_t rows, int64_t N, int row_bytes) {
@@ -110,6 +137,15 @@ constexpr int MAX_SPLIT_GROUPS = 16384;
 // launch meets in one XCD's L2 (1) or at device scope (0).
 hipError_t launch_partial(int fmt, int D, int hg, const PartialParams& p, int nblocks, int nw,
                           hipStream_t st, int* xcd_local = nullptr);
+// p.slot < 0 launches the piece merge as a second kernel.
+hipError_t launch_balanced(int fmt, int D, int hg, const BalancedParams& p, int nw, hipStream_t st,
+                           int* xcd_local = nullptr);
+// Waves per SIMD that decode_balanced_kernel is built for, and waves per
+// workgroup at most (the pieces of 16 heads fill the LDS at 8 waves).
+constexpr int balanced_waves(int fmt, int D, int hg) {
+  return D == 64 ? 4 : (fmt == 0 || fmt == 3 || hg == 16 ? 2 : 3);
+}
+constexpr int balanced_nw(int fmt, int D, int hg) { return balanced_waves(fmt, D, hg) == 2 ? 8 : 4; }
 // XCD period of a device as probed (> 0), 0 while not probed (or after a
 // probe that a HIP error cut short: it runs again on a later call), -1 when
 // the probe found no usable round-robin order.

@@ -349,3 +349,30 @@ def test_reference_quantizer_expressions_on_gpu_match_oracle(dtype, fmt):
         oq, os_ = oracle.quant_int8_per_token(X.numpy())
     np.testing.assert_array_equal(qv.cpu().numpy(), oq)
     np.testing.assert_array_equal(s.squeeze(-1).half().cpu().numpy().view(np.uint16), os_.view(np.uint16))
+
+
+@pytest.mark.parametrize("rows", [16383, 16384, 16385, 16417])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_gpu_narrow_rows_taken_two_at_a_time(dtype, rows):
+    """K and V rows around 32768 in all, D 64 (16-bit rows go two per lane group from there on, with
+    a remainder), and the plain form at twice as many: the bytes of the PyTorch expressions."""
+    g = torch.Generator().manual_seed(rows)
+    K = torch.randn(1, 1, rows, 64, generator=g).to(dtype).cuda()
+    V = torch.randn(1, 1, rows, 64, generator=g).to(dtype).cuda()
+    K[0, 0, -1] = 0
+    cap, pos = rows + 5, 3
+    kc = torch.full((1, 1, cap, 32), 0x5A, dtype=torch.uint8, device="cuda")
+    vc, ks = kc.clone(), torch.full((1, 1, cap), 7.0, dtype=torch.float16, device="cuda")
+    vs = ks.clone()
+    fq.quantize_kv_append_(K, V, kc, vc, ks, vs, pos)
+    src = (lambda x: x.float()) if dtype == torch.bfloat16 else (lambda x: x)
+    for x, c, s in ((K, kc, ks), (V, vc, vs)):
+        want, ws = quant.quant_int4_per_token(src(x))
+        assert torch.equal(c[:, :, pos:pos + rows], want)
+        assert torch.equal(s[:, :, pos:pos + rows].view(torch.int16), ws.view(torch.int16))
+        assert bool((c[:, :, :pos] == 0x5A).all()) and bool((c[:, :, pos + rows:] == 0x5A).all())
+        assert bool((s[:, :, :pos] == 7).all()) and bool((s[:, :, pos + rows:] == 7).all())
+    X = torch.cat([K, V], 2).reshape(-1, 64)
+    q, s = fq.quantize_int8_per_token(X)
+    want, ws = quant.quant_int8_per_token(src(X))
+    assert torch.equal(q, want) and torch.equal(s.view(torch.int16), ws.view(torch.int16))

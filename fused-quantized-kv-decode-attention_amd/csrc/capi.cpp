@@ -158,6 +158,10 @@ int device_cus(int* out) {
   return FQKV_OK;
 }
 
+int64_t row_bytes_of(int fmt, int64_t D) {
+  return (fmt == KV_F16 || fmt == KV_BF16) ? 2 * D : (fmt == KV_I4 ? D / 2 : D);
+}
+
 // Query heads per workgroup: the transposed-score kernels carry up to 16
 // heads in one matrix-core tile at the same cost, so a group takes all of
 // its KV row's query heads up to 16.
@@ -170,18 +174,44 @@ int choose_hg(int64_t G, int fmt) {
   return 16;
 }
 
-// Splits for the single-block entry points: about one workgroup per CU, each
-// split at least 32 tokens long (measured on MI355X over batch 1..256,
-// N 512..16K, G 1 and 4, W 4 and 8: more workgroups than CUs only adds merge
-// work; with two-tile passes for short splits, 32-token splits beat 64-token
-// ones where the cap binds: GQA B 1, N 512, D 64 5.16 -> 4.51 us).
-int64_t splits_for(int64_t rows, int64_t G, int64_t N, int fmt, int64_t W, int cus) {
-  (void)W;
+// Splits for the single-block entry points, each at least 32 tokens long
+// (measured on MI355X over batch 1..256, N 512..16K, G 1 and 4, W 4 and 8: more
+// workgroups than CUs only adds merge work; with two-tile passes for short
+// splits, 32-token splits beat 64-token ones where the cap binds: GQA B 1, N
+// 512, D 64 5.16 -> 4.51 us).
+//
+// Rows of one length (contiguous and strided caches): as many splits as fit one
+// round of a workgroup per CU. One split more leaves a second round nearly
+// empty, and a CU that got two workgroups sets the time. 8 waves, rounded up ->
+// down: 48 rows of 3001, bf16 D 128, 6 -> 5 splits 23.6 -> 17.8 us; 96 of 2500,
+// int8, 3 -> 2 25.1 -> 18.7; 160 of 3000, fp16, 2 -> 1 51.2 -> 40.7; 136 of 2000,
+// fp16 D 64, 2 -> 1 20.8 -> 15.2; 130 of 1000, int8 D 64, 2 -> 1 8.8 -> 7.6. Not
+// for 4 waves of int4 unsplit (160 rows 24.5 -> 28.4 us: too few bytes in
+// flight), nor for 2 waves, whose workgroups share a CU.
+// With a few more rows than CUs every CU but those few would idle for half of
+// the time: up to 4/3 rows per CU three splits are 4 rounds of a third (with 4
+// waves: less per workgroup to start and merge). fp16 D 128, 1 -> 3 splits, 264
+// rows of 2500 72.0 -> 62.4 us, 320 of 1777 57.1 -> 51.7, 340 of 2500 75.7 ->
+// 71.0; int8 D 128, 300 of 4000 69.5 -> 62.9; int4 D 128, 300 of 6000 53.4 ->
+// 48.9; beyond, 370 rows gain 3 % (fp16) or lose 5 % (fp8). Short rows do not
+// pay for the merge (300 of 400, fp16 17.2 -> 18.3; of 500, int8 12.9 -> 16.7
+// us), and 64-byte int8 / fp8 rows gain nothing (264 of 5000: 40.5 -> 47.3).
+//
+// Paged calls, whose lengths the host does not know, round up: a second round
+// is mostly workgroups with nothing to do where sequences are shorter than the
+// longest, which is what more splits cut.
+bool thirds_pay(int64_t groups, int64_t N, int64_t D, int fmt, int64_t W, int cus) {
+  const int64_t rowb = row_bytes_of(fmt, D);
+  if (W < 4 || groups <= cus || 3 * groups > 4LL * cus) return false;
+  return rowb >= 128 ? N >= 1536 : fmt == KV_I4 && N >= 4096;
+}
+int64_t splits_for(int64_t rows, int64_t G, int64_t N, int64_t D, int fmt, int64_t W, int cus, bool paged) {
   const int hg = choose_hg(G, fmt);
   const int64_t groups = rows * ((G + hg - 1) / hg);
   const int64_t target = (int64_t)cus;
-  if (groups >= target) return 1;
+  if (groups >= target) return !paged && thirds_pay(groups, N, D, fmt, W, cus) ? 3 : 1;
   int64_t S = (target + groups - 1) / groups;
+  if (!paged && (W == 8 || (W == 4 && !(fmt == KV_I4 && target / groups == 1)))) S = target / groups;
   const int64_t cap = N / 32;
   if (S > cap) S = cap;
   return S < 1 ? 1 : S;
@@ -203,9 +233,6 @@ int check_common(int64_t N, int64_t D, int64_t W) {
 
 // Single-block style decode: rows KV rows, G query heads per row. Splits the
 // sequence internally when rows alone cannot fill the GPU and the workspace allows.
-int64_t row_bytes_of(int fmt, int64_t D) {
-  return (fmt == KV_F16 || fmt == KV_BF16) ? 2 * D : (fmt == KV_I4 ? D / 2 : D);
-}
 // int8 / int4 / fp8: codes with per-token scales
 bool is_quant(int fmt) { return fmt == KV_I8 || fmt == KV_I4 || fmt == KV_FP8; }
 
@@ -338,8 +365,9 @@ int run_decode(int fmt, const void* q, const void* K, const void* V, const void*
   const int hg = choose_hg(G, fmt);
   const int64_t ngroups = (G + hg - 1) / hg;
   const int64_t heads = rows * G;
-  int64_t S = splits_for(rows, G, N, fmt, W, cus);
-  const bool balance = L && L->page_table &&
+  const bool paged = L && L->page_table;
+  int64_t S = splits_for(rows, G, N, D, fmt, W, cus, paged);
+  const bool balance = paged &&
                        balanced_pays(fmt, hg, rows / L->hkv, rows * ngroups, N, D, S, W, ws ? ws_bytes : 0, cus);
   if (balance) S = 1;
   if (S > 1 && (ws == nullptr || scratch_bytes(heads, S, D) > ws_bytes)) {
@@ -398,7 +426,8 @@ int run_decode(int fmt, const void* q, const void* K, const void* V, const void*
     p.o_part = f + acc_offset_floats(heads, S);
     p.slot = merge_slot(st, rows * ngroups, &p.xcd_ok);
   }
-  const int64_t nw = waves_for(fmt, D, nblocks, S, W, cus);
+  int64_t nw = waves_for(fmt, D, nblocks, S, W, cus);
+  if (S > 1 && !paged && rows * ngroups > cus && nw > 4) nw = 4;  // (see thirds_pay)
   int xcd_local = 0;
   hipError_t e = launch_partial(fmt, (int)D, hg, p, (int)nblocks, (int)nw, st, &xcd_local);
   if (e != hipSuccess) return hip_fail(e, "launch: partial kernel");
@@ -426,9 +455,6 @@ int check_ptrs_quant(int fmt, int64_t D, const void* q, const void* K, const voi
     return fail(FQKV_ERR_ARG, "q must be 16-byte aligned, o and scales 2-byte aligned");
   return FQKV_OK;
 }
-
-// The kernels address a KV row block with 32-bit byte offsets.
-int64_t row_bytes_of(int fmt, int64_t D);
 
 // Byte offsets inside a KV row are 32-bit, formed in the kernel as tile offset
 // + lane offset (for int4 summed by the load itself, the tile offset in the
@@ -590,19 +616,21 @@ int fqkv_device_cu_count(int* cu_count) {
 }
 
 int64_t fqkv_choose_splits(int64_t rows, int64_t G, int64_t N, int64_t D, int kv_format, int64_t W) {
-  (void)D;
   int cus = 256;
   if (device_cus(&cus) != FQKV_OK) cus = 256;
   if (rows < 1 || G < 1 || N < 1) return 1;
-  return splits_for(rows, G, N, kv_format, W, cus);
+  return splits_for(rows, G, N, D, kv_format, W, cus, false);
 }
 
 size_t fqkv_workspace_bytes(int64_t rows, int64_t G, int64_t N, int64_t D, int kv_format, int64_t W) {
   int cus = 256;
   if (device_cus(&cus) != FQKV_OK) cus = 256;
   if (rows < 1 || G < 1 || N < 1) return 0;
-  const int64_t S = splits_for(rows, G, N, kv_format, W, cus);
-  const size_t split = S > 1 ? scratch_bytes(rows * G, S, D) : 0;
+  // contiguous and paged calls of these sizes may split differently
+  const int64_t S = splits_for(rows, G, N, D, kv_format, W, cus, true);
+  const int64_t Sc = splits_for(rows, G, N, D, kv_format, W, cus, false);
+  const int64_t most = S > Sc ? S : Sc;
+  const size_t split = most > 1 ? scratch_bytes(rows * G, most, D) : 0;
   const int hg = choose_hg(G, kv_format);
   const int64_t work_rows = rows * ((G + hg - 1) / hg);
   // (a paged call of these sizes may take the work-balanced kernel)

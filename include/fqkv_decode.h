@@ -410,7 +410,7 @@ int fqkv_set_pv_valu(int enable);
 int fqkv_device_cu_count(int* cu_count);
 
 /*
- * Splits the single-block entry points use for a problem (1 = no split), as
+ * Splits the single-block entry points use for a contiguous cache (1 = no split), as
  * chosen from the current device's CU count; exposed for tests and tooling.
  */
 int64_t fqkv_choose_splits(int64_t rows, int64_t G, int64_t N, int64_t D, int kv_format,
